@@ -11,6 +11,26 @@ constexpr int kMaxVD = 12;  // VertexData floats of the widest fixed shader
 // Uniform block offsets (same layout as include/euchip.h documents).
 constexpr int U_VP = 0, U_L0 = 16, U_L1 = 20, U_CAM = 24, U_SURF = 28, U_K = 32, U_LPOS = 36, U_LVP = 40;
 
+// A device pointer kept in memory (a launch's parameters, a view).  Read in a
+// kernel it is a pointer to global memory: a plain pointer loaded from memory
+// could address anything, and the compiler would take FLAT instructions for it.
+template <class T>
+struct gptr {
+    T *ptr;
+    gptr &operator=(T *q) {
+        ptr = q;
+        return *this;
+    }
+    __host__ __device__ operator T *() const {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return (T *)(__attribute__((address_space(1))) T *)ptr;
+#else
+        return ptr;
+#endif
+    }
+    __host__ __device__ T *operator->() const { return *this; }
+};
+
 enum Shader : uint32_t { FLAT = 0, COLOR = 1, GOURAUD = 2, PHONG = 3, DEPTH_ONLY = 4, TEXTURED = 5, PHONG_SHADOW = 6, TEX_SHADOW = 7 };
 enum DepthTest : uint32_t { DT_NONE = 0, DT_LESS = 1, DT_EQUAL = 2, DT_GREATER = 3 };
 
@@ -153,24 +173,24 @@ struct View {
     uint32_t tri_base;     // first triangle of this request in rec0 / rec1
     uint32_t tile_cap;     // bin slots per tile of this request
     uint64_t bin_base;     // first bin slot of this request
-    uint32_t *pixel;
-    float *depth;
+    gptr<uint32_t> pixel;
+    gptr<float> depth;
     uint32_t clear_color_en, clear_color, clear_depth_en;
     float clear_depth;
     float ndc_x, ndc_y;    // 2/size_x and -2/size_y of to_ndc (triangles.rs:44-48)
     // mesh (device)
-    const float *pos;
-    const float *nrm;
-    const float *col;
-    const float *uv;
-    const uint32_t *rgba8;
-    const uint32_t *idx;
-    const float *models;
+    gptr<const float> pos;
+    gptr<const float> nrm;
+    gptr<const float> col;
+    gptr<const float> uv;
+    gptr<const uint32_t> rgba8;
+    gptr<const uint32_t> idx;
+    gptr<const float> models;
     uint32_t pos_comps, count, n_vertices, n_instances, n_tris;
     // textures (device)
-    const uint32_t *tex;
+    gptr<const uint32_t> tex;
     uint32_t tex_w, tex_h;
-    const float *shadow;
+    gptr<const float> shadow;
     uint32_t sh_w, sh_h;
     float u[kUniforms];
 };
@@ -191,20 +211,20 @@ struct FrameParams {
     // lines (one-request frames): LINE_LIST or LINE_TRIANGLE_LIST, n_lines lines;
     // a 64-byte record per line and a 64-bit winner key per target pixel
     uint32_t primitives, n_lines;
-    uint32_t *lrec;
-    uint64_t *lkey;
+    gptr<uint32_t> lrec;
+    gptr<uint64_t> lkey;
     // per-launch scratch (device)
-    uint4 *rec0;           // kRec0Quads per triangle of the launch
-    uint4 *rec1;           // kRec1Quads per triangle of the launch
-    float *vary;           // VertexData per shaded vertex
-    Counters *ctr;
-    TileBin *tile_count;   // per tile of the launch, zero before setup, read-only in raster
-    uint32_t *bins;        // bin_base + local tile * tile_cap + rank -> primitive
-    uint32_t *req_max;     // batches, per request: largest tile count above its tile_cap (host grows the bins)
-    uint32_t *pool;        // overflow segments (ranks >= tile_cap), pool_cap words
+    gptr<uint4> rec0;           // kRec0Quads per triangle of the launch
+    gptr<uint4> rec1;           // kRec1Quads per triangle of the launch
+    gptr<float> vary;           // VertexData per shaded vertex
+    gptr<Counters> ctr;
+    gptr<TileBin> tile_count;   // per tile of the launch, zero before setup, read-only in raster
+    gptr<uint32_t> bins;        // bin_base + local tile * tile_cap + rank -> primitive
+    gptr<uint32_t> req_max;     // batches, per request: largest tile count above its tile_cap (host grows the bins)
+    gptr<uint32_t> pool;        // overflow segments (ranks >= tile_cap), pool_cap words
     uint32_t pool_cap;
-    Report *report;        // host-visible report of one-request frames, or null
-    uint32_t *heavy;       // tiles with at least kHeavyTile entries (heavy_cap slots)
+    gptr<Report> report;        // host-visible report of one-request frames, or null
+    gptr<uint32_t> heavy;       // tiles with at least kHeavyTile entries (heavy_cap slots)
     uint32_t heavy_cap;    // 0: no heavy-first pass
     // Setup lists the tiles it bins into (busy) in 8 lists of up to ntiles
     // entries (list x at busy + x * ntiles, chosen by busy_map); raster clears
@@ -212,9 +232,9 @@ struct FrameParams {
     // `tile_count` as it is and zeroes the first `zero_n` counts of
     // `count_next` (one-request frames: the other half of a two-frame count
     // buffer; batches zero their counts with a fill before setup).
-    uint32_t *busy;
+    gptr<uint32_t> busy;
     uint32_t busy_map;
-    uint32_t *big;         // big triangles (primitive ids), big_cap slots; big_cap 0: off (batches)
+    gptr<uint32_t> big;         // big triangles (primitive ids), big_cap slots; big_cap 0: off (batches)
     uint32_t big_cap;
     // Row checkpoints (ck_on): per triangle its big record (kBigRecQuads
     // quads), the pool of n_tris x ntx x H slots and the tiles' lists
@@ -226,24 +246,24 @@ struct FrameParams {
     // blocks up to setup_blocks; a checkpoint frame's has setup_blocks blocks
     // of triangles and vertices, then the span blocks (span_parts items of
     // kSpanRows rows per triangle, 4 per block).
-    uint4 *big_rec;
-    uint4 *ck;
+    gptr<uint4> big_rec;
+    gptr<uint4> ck;
     uint32_t ck_on;
-    uint2 *cktab;
+    gptr<uint2> cktab;
     uint32_t mstride;
-    uint2 *ck_count, *ck_count_next;  // per tile (list length, ~least occluder bound)
+    gptr<uint2> ck_count, ck_count_next;  // per tile (list length, ~least occluder bound)
     uint32_t ck_zero_n;
     uint32_t tri_blocks, setup_blocks, span_parts;
-    TileBin *count_next;
+    gptr<TileBin> count_next;
     uint32_t zero_n;
     uint32_t frame;        // frame parity selects the overflow counter and tile queue
     uint32_t ntiles;       // tiles of all requests
     uint32_t tile_sx;      // tiles are (1 << tile_sx) x (256 >> tile_sx) pixels, tile_sx in 3..5
     // requests: one in `v0` (kernel argument), or `n_views` in device memory
     uint32_t n_views;
-    const View *views;
-    const uint2 *blk;          // batched setup: workgroup -> (request, workgroup within the request)
-    const uint32_t *tile_req;  // batched raster: tile -> request
+    gptr<const View> views;
+    gptr<const uint2> blk;          // batched setup: workgroup -> (request, workgroup within the request)
+    gptr<const uint32_t> tile_req;  // batched raster: tile -> request
     View v0;
 };
 

@@ -37,6 +37,35 @@ namespace euchip {
 
 EUCHIP_DEV uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
+// The launch's parameters, read anew from the kernel argument segment: the
+// kernels take one reference per phase of their work.  The address passes
+// through an empty asm, so a value loaded for one phase is not kept in a
+// register through the others (a uniform value that did not fit the scalar
+// registers went to vector-register lanes, and every use of it took a
+// v_readlane: a quarter of the raster kernels' vector instructions).  Scalar
+// loads of a line that the scalar cache holds cost no vector issue at all.
+#define EUCHIP_CONST __attribute__((address_space(4)))
+EUCHIP_DEV const FrameParams &args() {
+    const EUCHIP_CONST FrameParams *k = (const EUCHIP_CONST FrameParams *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    return *(const FrameParams *)__builtin_assume_aligned((const FrameParams *)k, 16);
+}
+
+// Bring every line of the parameters into the scalar cache, all in flight at
+// once, when a kernel starts: a phase that met its lines cold would wait for
+// them again.
+EUCHIP_DEV void warm_args() {
+    const EUCHIP_CONST uint32_t *k = (const EUCHIP_CONST uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr uint32_t lines = (sizeof(FrameParams) + 63u) / 64u;
+    static_assert(lines <= 16u, "one load per line below");
+#define EUCHIP_LINE(i) k[16u * (i < lines ? i : lines - 1u)]
+    asm volatile("" ::"s"(EUCHIP_LINE(0)), "s"(EUCHIP_LINE(1)), "s"(EUCHIP_LINE(2)), "s"(EUCHIP_LINE(3)),
+                 "s"(EUCHIP_LINE(4)), "s"(EUCHIP_LINE(5)), "s"(EUCHIP_LINE(6)), "s"(EUCHIP_LINE(7)),
+                 "s"(EUCHIP_LINE(8)), "s"(EUCHIP_LINE(9)), "s"(EUCHIP_LINE(10)), "s"(EUCHIP_LINE(11)),
+                 "s"(EUCHIP_LINE(12)), "s"(EUCHIP_LINE(13)), "s"(EUCHIP_LINE(14)), "s"(EUCHIP_LINE(15)));
+#undef EUCHIP_LINE
+}
+
 EUCHIP_DEV bool passes_z_clip(const FrameParams &p, float z) {
     return !p.z_clip || (p.z_min <= z && z <= p.z_max);
 }
@@ -341,11 +370,22 @@ EUCHIP_DEV void bin_direct(const FrameParams &p, const View &v, uint32_t tile, u
 }
 
 // The request a workgroup or tile works on: the kernel argument's, or one of
-// the batch's in device memory.
+// the batch's in device memory, which no kernel writes: read as constants, by
+// scalar loads (r is uniform), and anew for each phase like the parameters.
 template <bool BATCH>
 EUCHIP_DEV const View &view_of(const FrameParams &p, uint32_t r) {
-    if constexpr (BATCH) return p.views[r];
-    else return p.v0;
+    if constexpr (BATCH) {
+        const EUCHIP_CONST View *k = (const EUCHIP_CONST View *)(const View *)p.views + r;
+        asm volatile("" : "+s"(k));
+        return *(const View *)__builtin_assume_aligned((const View *)k, 8);
+    } else {
+        return p.v0;
+    }
+}
+
+// The key mode of the frame's depth rule (see init_key).
+EUCHIP_DEV uint32_t key_mode(const FrameParams &p) {
+    return (p.depth_write && p.depth_test == DT_LESS) ? 1u : (p.depth_write && p.depth_test == DT_GREATER) ? 2u : 0u;
 }
 
 // Stores that bypass the caches on their way to memory: setup records (read
@@ -483,7 +523,9 @@ union SetupShared {
 // SPAN: the launch of a checkpoint frame, whose blocks past setup_blocks are
 // span blocks (compiled apart so other frames' setup carries none of their code).
 template <uint32_t SH, bool BATCH, bool SPAN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_setup(FrameParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_setup(FrameParams) {
+    warm_args();
+    const FrameParams &p = args();
     __shared__ SetupShared sm;
     __shared__ uint32_t npl;
     __shared__ uint32_t lcnt[9], lbase[9];  // new busy tiles per list (8) and new heavy tiles (8)
@@ -509,7 +551,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     uint32_t r = 0, j = blockIdx.x;
     if constexpr (BATCH) {
         const uint2 bj = p.blk[blockIdx.x];
-        r = bj.x, j = bj.y;
+        r = __builtin_amdgcn_readfirstlane(bj.x), j = __builtin_amdgcn_readfirstlane(bj.y);
     }
     const View &v = view_of<BATCH>(p, r);
     const uint32_t t = j * 256u + tid;
@@ -986,17 +1028,17 @@ struct TileShared {
 };
 
 // Rows of bin entry `prim` inside the tile, its setup kept in sh.tri[slot].
-EUCHIP_DEV uint32_t stage_entry(const FrameParams &p, const View &v, TileShared &sh, uint32_t slot, uint32_t prim,
+EUCHIP_DEV uint32_t stage_entry(const FrameParams &p, uint32_t tri_base, TileShared &sh, uint32_t slot, uint32_t prim,
                                 const TileGeom &g) {
     TriRec R;
-    load_rec0(p, v.tri_base + prim, R);
+    load_rec0(p, tri_base + prim, R);
     const uint32_t ry0 = R.ymin > g.Y0 ? R.ymin : g.Y0;
     const uint32_t ry1 = R.ymax < g.Y0 + g.TH ? R.ymax : g.Y0 + g.TH;
     const uint32_t xs = R.xmin > g.X0 ? R.xmin : g.X0;
     const uint32_t xe = R.xmax < g.X0 + g.TW ? R.xmax : g.X0 + g.TW;
     if (ry0 >= ry1 || xs >= xe) return 0u;
     if (!all_rows_boxed(R)) {
-        load_rec1(p, v.tri_base + prim, R);
+        load_rec1(p, tri_base + prim, R);
     } else {
 #pragma unroll
         for (int i = 0; i < 6; i++) R.vby[i] = 0.0f;  // boxed rows never read verts_by_y
@@ -1024,9 +1066,11 @@ EUCHIP_DEV uint32_t block_inclusive_sum(TileShared &sh, uint32_t tid, uint32_t v
 // then the (entry, row) pairs of the batch are spread over all lanes so no
 // lane walks much more than one row.
 template <bool OWNER, bool LONG_ROWS>
-EUCHIP_DEV void raster_batch(const FrameParams &p, const View &v, TileShared &sh, uint32_t tid, bool valid,
-                             uint32_t prim, const TileGeom &g, uint32_t mode) {
-    const uint32_t rows = valid ? stage_entry(p, v, sh, tid, prim, g) : 0u;
+EUCHIP_DEV void raster_batch(uint32_t tri_base, TileShared &sh, uint32_t tid, bool valid, uint32_t prim,
+                             const TileGeom &g) {
+    const FrameParams &p = args();
+    const uint32_t mode = key_mode(p);
+    const uint32_t rows = valid ? stage_entry(p, tri_base, sh, tid, prim, g) : 0u;
     const uint32_t incl = block_inclusive_sum(sh, tid, rows);
     const uint32_t excl = incl - rows;
     sh.rows_incl[tid] = incl;
@@ -1081,7 +1125,8 @@ struct BigTaskLds {
 static_assert(sizeof(BigTaskLds) <= sizeof(TriLds) * kBatch, "big-triangle tasks fit the staging space");
 
 EUCHIP_DEV void big_tasks(const FrameParams &p, TileShared &sh, uint32_t tid, uint32_t tile, uint32_t nbig,
-                          uint32_t occl, const TileGeom &g, uint32_t mode, uint2 e_first) {
+                          uint32_t occl, const TileGeom &g, uint2 e_first) {
+    const uint32_t mode = key_mode(p);
     BigTaskLds &bt = *reinterpret_cast<BigTaskLds *>(sh.tri);
     const uint2 *list = p.cktab + (size_t)tile * p.mstride;
     const uint4 *cktile = p.ck + (size_t)(g.X0 >> g.sx) * p.v0.H + g.Y0;  // triangle t's at + t * ntx * H
@@ -1145,64 +1190,72 @@ constexpr uint32_t raster_waves(uint32_t sh, bool ms, bool big) {
 }
 
 template <uint32_t SH, bool BATCH, bool BIG, bool GS, bool MS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(SH, MS, BIG)))) void k_raster(FrameParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(SH, MS, BIG)))) void k_raster(FrameParams) {
     __shared__ TileShared sh;
+    warm_args();
     const uint32_t tid = threadIdx.x;
-    const uint32_t ntiles = p.ntiles;
-    const uint32_t par = p.frame & 1u, npar = (p.frame + 1u) & 1u;
     const uint32_t xcd = blockIdx.x & 7u;
     const uint32_t per_xcd = gridDim.x >> 3, w = blockIdx.x >> 3;
-    // The loads the first tile waits for, issued together: frame flags, pool use,
-    // list lengths, this workgroup's first busy tile and its bin state (read at a
-    // clamped index before the tile is known to be in the list; used only if it is).
-    uint32_t lbase, lcap;
-    busy_list_span(p, xcd, lbase, lcap);
-    const uint32_t *list = p.busy + lbase;  // this XCD's busy list
-    const uint32_t flags = p.ctr->flags[par][0];
-    const uint32_t pool_used0 = p.ctr->pool[par][0];
-    uint32_t nh = __builtin_amdgcn_readfirstlane(p.ctr->heavy[par][0]);
-    // big triangles (with checkpoints any triangle may be on any tile's list)
-    uint32_t nbig = !BIG ? 0u : p.ck_on ? p.v0.n_tris : __builtin_amdgcn_readfirstlane(p.ctr->big[par][0]);
-    uint32_t nbusy = __builtin_amdgcn_readfirstlane(p.ctr->busy[par][xcd][0]);
-    const uint32_t first = w < lcap ? __builtin_amdgcn_readfirstlane(list[w]) : 0u;
-    const TileBin first_bin = p.tile_count[first < ntiles ? first : 0u];
-    if (p.report && blockIdx.x == 0u && tid == 0u) {
-        // this frame's setup counts, for the host (frame number last)
-        Report *rp = p.report;
-        rp->max_count = p.ctr->max_count[par][0];
-        rp->flags = flags;
-        rp->pool_used = pool_used0;
-        if (flags & FLAG_BIN_OVERFLOW) rp->dropped = rp->dropped + 1u;
-        __threadfence_system();
-        rp->frame = p.frame;
+    uint32_t nh, nbusy, nbig, first, pool_used;
+    TileBin first_bin;
+    {
+        const FrameParams &p = args();
+        const uint32_t par = p.frame & 1u, npar = (p.frame + 1u) & 1u;
+        // The loads the first tile waits for, issued together: frame flags, pool use,
+        // list lengths, this workgroup's first busy tile and its bin state (read at a
+        // clamped index before the tile is known to be in the list; used only if it is).
+        uint32_t lbase, lcap;
+        busy_list_span(p, xcd, lbase, lcap);
+        const uint32_t flags = p.ctr->flags[par][0];
+        pool_used = p.ctr->pool[par][0];
+        nh = __builtin_amdgcn_readfirstlane(p.ctr->heavy[par][0]);
+        // big triangles (with checkpoints any triangle may be on any tile's list)
+        nbig = !BIG ? 0u : p.ck_on ? p.v0.n_tris : __builtin_amdgcn_readfirstlane(p.ctr->big[par][0]);
+        nbusy = __builtin_amdgcn_readfirstlane(p.ctr->busy[par][xcd][0]);
+        first = w < lcap ? __builtin_amdgcn_readfirstlane(p.busy[lbase + w]) : 0u;
+        first_bin = p.tile_count[first < p.ntiles ? first : 0u];
+        if (p.report && blockIdx.x == 0u && tid == 0u) {
+            // this frame's setup counts, for the host (frame number last)
+            Report *rp = p.report;
+            rp->max_count = p.ctr->max_count[par][0];
+            rp->flags = flags;
+            rp->pool_used = pool_used;
+            if (flags & FLAG_BIN_OVERFLOW) rp->dropped = rp->dropped + 1u;
+            __threadfence_system();
+            rp->frame = p.frame;
+        }
+        // The next frame's counters start at zero (its setup counts into them).
+        if (blockIdx.x == 0u && tid == 0u) {
+            p.ctr->pool[npar][0] = 0u;
+            p.ctr->flags[npar][0] = 0u;
+            p.ctr->max_count[npar][0] = 0u;
+            p.ctr->heavy[npar][0] = 0u;
+            p.ctr->big[npar][0] = 0u;
+        }
+        if (blockIdx.x < 8u && tid == 0u) {
+            p.ctr->next[npar][xcd][0] = 0u;
+            p.ctr->empty[npar][xcd][0] = 0u;
+            p.ctr->busy[npar][xcd][0] = 0u;
+        }
+        for (uint32_t i = blockIdx.x * 256u + tid; i < p.zero_n; i += gridDim.x * 256u) p.count_next[i] = TileBin{0u, 0u};
+        if constexpr (BIG)  // after a checkpoint frame: its list counts
+            for (uint32_t i = blockIdx.x * 256u + tid; i < p.ck_zero_n; i += gridDim.x * 256u)
+                p.ck_count_next[i] = make_uint2(0u, 0u);
+        // The pool ran out in setup: entries were lost, the frame is dropped (the
+        // host sees the flag and re-runs it with a larger pool).
+        if (flags & FLAG_BIN_OVERFLOW) return;
+        pool_used = pool_used < p.pool_cap ? pool_used : p.pool_cap;
+        if (BIG && !p.ck_on) nbig = nbig < p.big_cap ? nbig : p.big_cap;
+        // With big triangles every tile may hold fragments: the loop below then takes
+        // every tile of this XCD's contiguous range instead of its busy list.
+        if (BIG && nbig) {
+            uint32_t b0, b1;
+            xcd_range(p.ntiles, xcd, b0, b1);
+            nbusy = b1 - b0;
+        }
+        nh = nh < p.heavy_cap ? nh : p.heavy_cap;
+        nbusy = nbusy < lcap ? nbusy : lcap;
     }
-    // The next frame's counters start at zero (its setup counts into them).
-    if (blockIdx.x == 0u && tid == 0u) {
-        p.ctr->pool[npar][0] = 0u;
-        p.ctr->flags[npar][0] = 0u;
-        p.ctr->max_count[npar][0] = 0u;
-        p.ctr->heavy[npar][0] = 0u;
-        p.ctr->big[npar][0] = 0u;
-    }
-    if (blockIdx.x < 8u && tid == 0u) {
-        p.ctr->next[npar][xcd][0] = 0u;
-        p.ctr->empty[npar][xcd][0] = 0u;
-        p.ctr->busy[npar][xcd][0] = 0u;
-    }
-    for (uint32_t i = blockIdx.x * 256u + tid; i < p.zero_n; i += gridDim.x * 256u) p.count_next[i] = TileBin{0u, 0u};
-    if constexpr (BIG)  // after a checkpoint frame: its list counts
-        for (uint32_t i = blockIdx.x * 256u + tid; i < p.ck_zero_n; i += gridDim.x * 256u) p.ck_count_next[i] = make_uint2(0u, 0u);
-    // The pool ran out in setup: entries were lost, the frame is dropped (the
-    // host sees the flag and re-runs it with a larger pool).
-    if (flags & FLAG_BIN_OVERFLOW) return;
-    const uint32_t pool_used = pool_used0 < p.pool_cap ? pool_used0 : p.pool_cap;
-    const bool uses_depth = p.depth_test != DT_NONE || p.depth_write;
-    const uint32_t mode = (p.depth_write && p.depth_test == DT_LESS) ? 1u
-                        : (p.depth_write && p.depth_test == DT_GREATER) ? 2u : 0u;
-    const uint32_t sx = p.tile_sx, sy = 8u - sx;
-    uint32_t *next = &p.ctr->next[par][xcd][0];
-    // big triangles from their row checkpoints (else walked from the row starts)
-    const bool ckp = BIG && p.ck_on;
 
     // One tile with `cnt` bin entries and overflow list `head`: winner keys in
     // LDS, then the resolve.
@@ -1213,40 +1266,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         // Batches (hundreds of tiles per workgroup) take the next queue index
         // when the tile starts and load that tile's list entry and bin state
         // before the resolve, so the next tile starts with no load to wait for.
-        uint32_t claimed = 0u;
-        if (BATCH && claim && tid == 0u) claimed = per_xcd + atomicAdd(next, 1u);
-        uint32_t r = 0;
-        if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(p.tile_req[tile]);
-        const View &v = view_of<BATCH>(p, r);
-        const uint32_t lt = tile - v.tile_base;
-        const uint32_t ty = lt / v.ntx, tx = lt - ty * v.ntx;
+        uint32_t claimed = 0u, r = 0u, lt, sx, nck = 0u, occl = 0u, run, nb, tri_base;
+        uint64_t bin_at;  // first bin slot of the tile
+        uint32_t seg = 0u;
         TileGeom g;
-        g.sx = sx, g.TW = 1u << sx, g.TH = 256u >> sx;
-        g.X0 = tx << sx, g.Y0 = ty << sy;
-        const uint32_t px = g.X0 + (tid & (g.TW - 1u)), py = g.Y0 + (tid >> sx);
-        const bool inside = px < v.W && py < v.H;
-        const size_t pidx = (size_t)py * v.W + px;
-        float D0 = 0.0f;
-        if (inside && uses_depth) D0 = v.clear_depth_en ? v.clear_depth : v.depth[pidx];
-        const uint32_t lp = tid + (tid >> sx);  // padded LDS index of this lane's pixel
-        sh.key[lp] = init_key(mode, D0);
-        sh.d0s[lp] = D0;
-        if (tid < g.TH) {
-            uint32_t by0, by1;
-            band_of(p, v, g.Y0 + tid, by0, by1);
-            sh.band[2 * tid] = by0;
-            sh.band[2 * tid + 1] = by1;
-        }
-        const uint32_t cap = v.tile_cap;
-        const uint32_t *bin = p.bins + v.bin_base + (size_t)lt * cap;
-        // the tile's checkpoint list: its length and first 256 entries, loaded
-        // now (used after the bin; entries past the length are ignored)
-        uint32_t nck = 0u, occl = 0u;
         uint2 e_first = make_uint2(0u, 0u);
-        if (BIG && ckp) {
-            const uint2 cc = p.ck_count[tile];
-            nck = cc.x, occl = ~cc.y;
-            if (tid < p.mstride) e_first = p.cktab[(size_t)tile * p.mstride + tid];
+        bool ckp = false;  // big triangles from their row checkpoints (else walked from the row starts)
+        {
+            const FrameParams &p = args();
+            if (BATCH && claim && tid == 0u) claimed = per_xcd + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
+            if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(p.tile_req[tile]);
+            const View &v = view_of<BATCH>(p, r);
+            lt = tile - v.tile_base;
+            const uint32_t ty = lt / v.ntx, tx = lt - ty * v.ntx;
+            sx = p.tile_sx;
+            g.sx = sx, g.TW = 1u << sx, g.TH = 256u >> sx;
+            g.X0 = tx << sx, g.Y0 = ty << (8u - sx);
+            const uint32_t px = g.X0 + (tid & (g.TW - 1u)), py = g.Y0 + (tid >> sx);
+            float D0 = 0.0f;
+            if ((p.depth_test != DT_NONE || p.depth_write) && px < v.W && py < v.H)
+                D0 = v.clear_depth_en ? v.clear_depth : v.depth[(size_t)py * v.W + px];
+            const uint32_t lp = tid + (tid >> sx);  // padded LDS index of this lane's pixel
+            sh.key[lp] = init_key(key_mode(p), D0);
+            sh.d0s[lp] = D0;
+            if (tid < g.TH) {
+                uint32_t by0, by1;
+                band_of(p, v, g.Y0 + tid, by0, by1);
+                sh.band[2 * tid] = by0;
+                sh.band[2 * tid + 1] = by1;
+            }
+            const uint32_t cap = v.tile_cap;
+            tri_base = v.tri_base;
+            bin_at = v.bin_base + (uint64_t)lt * cap;
+            nb = cnt < cap ? cnt : cap;
+            seg = cnt > cap ? head : 0u;
+            // the tile's checkpoint list: its length and first 256 entries, loaded
+            // now (used after the bin; entries past the length are ignored)
+            if constexpr (BIG) {
+                ckp = p.ck_on;
+                if (ckp) {
+                    const uint2 cc = p.ck_count[tile];
+                    nck = cc.x, occl = ~cc.y;
+                    if (tid < p.mstride) e_first = p.cktab[(size_t)tile * p.mstride + tid];
+                }
+            }
+            run = nb + (ckp ? 0u : nbig);  // entries of the current run
         }
         __syncthreads();
         // Runs of entries, kBatch at a time: this tile's bin and the big
@@ -1255,19 +1319,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         // in this frame, each pointing at the one taken before it; a walk of at
         // most pool_used / 3 segments whose every read stays below pool_used
         // ends even on a damaged list.  One loop, so one copy of raster_batch.
-        const uint32_t nb = cnt < cap ? cnt : cap;
-        uint32_t run = nb + (ckp ? 0u : nbig);  // entries of the current run
         uint32_t base = 0u;                 // pool index of the current segment's entries (0: bin + big)
-        uint32_t seg = cnt > cap ? head : 0u, guard = 0u;
+        uint32_t guard = 0u;
         for (uint32_t b = 0;; b += kBatch) {
             while (b >= run) {              // next segment (uniform)
                 if (!seg || guard++ > pool_used / 3u || seg + 1u > pool_used) {
                     seg = 0u;
                     break;
                 }
+                const uint32_t *pool = args().pool;
                 const uint32_t s0 = seg - 1u;
-                seg = __builtin_amdgcn_readfirstlane(p.pool[s0]);
-                const uint32_t len = __builtin_amdgcn_readfirstlane(p.pool[s0 + 1u]);
+                seg = __builtin_amdgcn_readfirstlane(pool[s0]);
+                const uint32_t len = __builtin_amdgcn_readfirstlane(pool[s0 + 1u]);
                 base = s0 + 2u;
                 run = len < pool_used - base ? len : pool_used - base;
                 b = 0u;
@@ -1278,43 +1341,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             uint32_t prim = 0;
             if (tid >= kBatch || i >= run) {
             } else if (base) {
-                valid = true, prim = p.pool[base + i];
+                // (read once; a plain load would be merged with the bin's into one FLAT load)
+                valid = true, prim = __builtin_nontemporal_load(&args().pool[base + i]);
             } else if (i < nb) {
-                valid = true, prim = bin[i];
+                valid = true, prim = args().bins[bin_at + i];
             } else if constexpr (BIG) {
-                valid = true, prim = p.big[i - nb];
+                valid = true, prim = args().big[i - nb];
             }
-            raster_batch<!BATCH, BIG>(p, v, sh, tid, valid, prim, g, mode);
+            raster_batch<!BATCH, BIG>(tri_base, sh, tid, valid, prim, g);
         }
         if (BIG && ckp) {
             nck = __builtin_amdgcn_readfirstlane(nck);
-            if (nck) big_tasks(p, sh, tid, tile, nck, __builtin_amdgcn_readfirstlane(occl), g, mode, e_first);
+            if (nck) big_tasks(args(), sh, tid, tile, nck, __builtin_amdgcn_readfirstlane(occl), g, e_first);
         }
         uint32_t ntile = 0u;
         TileBin ntb{0u, 0u};
-        if (BATCH && claim && tid == 0u && claimed < nbusy) {
-            ntile = list[claimed];
-            ntb = p.tile_count[ntile];
-        }
-        if (!BATCH && claim && tid == 0u) claimed = per_xcd + atomicAdd(next, 1u);
         bool shade = false;  // this lane's pixel has a winner to shade
-        if (inside) {
-            const uint64_t kk = sh.key[lp];
-            bool has;  // a winner (its primitive is read again by the shading lanes)
-            float z;
-            if (mode == 0u) {
-                has = kk != 0ull;
-                z = __uint_as_float((uint32_t)kk);
-            } else {
-                has = ((uint32_t)kk) != 0u;
-                const uint32_t o = (uint32_t)(kk >> 32);
-                z = zunord(mode == 1u ? o : ~o, (uint32_t)kk & 1u);
+        {
+            const FrameParams &p = args();
+            const View &v = view_of<BATCH>(p, r);
+            const uint32_t mode = key_mode(p);
+            if (BATCH && claim && tid == 0u && claimed < nbusy) {
+                uint32_t lbase, lcap;
+                busy_list_span(p, xcd, lbase, lcap);
+                ntile = p.busy[lbase + claimed];
+                ntb = p.tile_count[ntile];
             }
-            shade = v.pixel && p.pixel_write && has && SH != DEPTH_ONLY;
-            if (v.pixel && !shade && v.clear_color_en) store_stream(&v.pixel[pidx], v.clear_color);
-            if (v.depth) {
-                if (has && p.depth_write) store_stream(&v.depth[pidx], z);
-                else if (v.clear_depth_en) store_stream(&v.depth[pidx], v.clear_depth);
+            if (!BATCH && claim && tid == 0u) claimed = per_xcd + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
+            const uint32_t px = g.X0 + (tid & (g.TW - 1u)), py = g.Y0 + (tid >> sx);
+            if (px < v.W && py < v.H) {
+                const size_t pidx = (size_t)py * v.W + px;
+                const uint64_t kk = sh.key[tid + (tid >> sx)];
+                bool has;  // a winner (its primitive is read again by the shading lanes)
+                float z;
+                if (mode == 0u) {
+                    has = kk != 0ull;
+                    z = __uint_as_float((uint32_t)kk);
+                } else {
+                    has = ((uint32_t)kk) != 0u;
+                    const uint32_t o = (uint32_t)(kk >> 32);
+                    z = zunord(mode == 1u ? o : ~o, (uint32_t)kk & 1u);
+                }
+                shade = v.pixel && p.pixel_write && has && SH != DEPTH_ONLY;
+                if (v.pixel && !shade && v.clear_color_en) store_stream(&v.pixel[pidx], v.clear_color);
+                if (v.depth) {
+                    if (has && p.depth_write) store_stream(&v.depth[pidx], z);
+                    else if (v.clear_depth_en) store_stream(&v.depth[pidx], v.clear_depth);
+                }
             }
         }
         // The pixels to shade, packed onto the first lanes in tile order: a wave
@@ -1333,12 +1406,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             if (shade) sh.owner[at + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = (uint8_t)tid;
             __syncthreads();
             if (tid < total) {
+                const FrameParams &p = args();
+                const View &v = view_of<BATCH>(p, r);
                 const uint32_t t = sh.owner[tid];
                 const uint32_t tx2 = g.X0 + (t & (g.TW - 1u)), ty2 = g.Y0 + (t >> sx);
                 const uint64_t kk = sh.key[t + (t >> sx)];
-                const uint32_t prim = mode == 0u ? (uint32_t)(kk >> 32) - 1u : ((uint32_t)kk >> 1) - 1u;
+                const uint32_t prim = key_mode(p) == 0u ? (uint32_t)(kk >> 32) - 1u : ((uint32_t)kk >> 1) - 1u;
                 TriRec R;
-                load_rec0(p, v.tri_base + prim, R);
+                load_rec0(p, tri_base + prim, R);
                 tri_sids(v, p.geometry, prim, R.flags, R.sid);
                 store_stream(&v.pixel[(size_t)ty2 * v.W + tx2],
                              shade_pixel<SH, GS, MS>(p, v, R, tx2, ty2, sh.band[2 * (t >> sx)],
@@ -1352,61 +1427,60 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         __syncthreads();
     };
 
-    if (BIG && !p.ck_on) nbig = nbig < p.big_cap ? nbig : p.big_cap;
-    // With big triangles every tile may hold fragments: the loop below then takes
-    // every tile of this XCD's contiguous range instead of its busy list.
-    if (BIG && nbig) {
-        uint32_t b0, b1;
-        xcd_range(ntiles, xcd, b0, b1);
-        nbusy = b1 - b0;
-    }
-    nh = nh < p.heavy_cap ? nh : p.heavy_cap;
-    nbusy = nbusy < lcap ? nbusy : lcap;
-    // 1. Heavy tiles first, workgroup k taking heavy[k] (the longest tiles
-    //    start early instead of ending the launch late).
-    for (uint32_t k = blockIdx.x; k < nh; k += gridDim.x) {
-        const uint32_t tile = __builtin_amdgcn_readfirstlane(p.heavy[k]);
-        const TileBin tb = p.tile_count[tile];
-        run_tile(tile, __builtin_amdgcn_readfirstlane(tb.count), __builtin_amdgcn_readfirstlane(tb.head), false);
-    }
-    // 2. Busy tiles of this XCD's list: the first by workgroup index, the rest
-    //    from the XCD's counter (heavy ones are done).
-    for (uint32_t k = w; k < nbusy;) {
+    // Heavy tiles first, workgroup k taking heavy[k] (the longest tiles start
+    // early instead of ending the launch late); then the busy tiles of this XCD's
+    // list: the first by workgroup index, the rest from the XCD's counter (heavy
+    // ones are done).  One loop, so one copy of the tile code.
+    for (uint32_t hk = blockIdx.x, k = w;;) {
+        const bool heavy = hk < nh;
+        if (!heavy && k >= nbusy) break;
+        const FrameParams &p = args();
         uint32_t tile;
-        if (BIG && nbig) {
+        TileBin tb;
+        if (heavy) {
+            tile = __builtin_amdgcn_readfirstlane(p.heavy[hk]);
+            tb = p.tile_count[tile];
+            hk += gridDim.x;
+        } else if (BIG && nbig) {
             uint32_t b0, b1;
-            xcd_range(ntiles, xcd, b0, b1);
+            xcd_range(p.ntiles, xcd, b0, b1);
             tile = b0 + k;
-        } else if (BATCH && k != w) {
-            tile = __builtin_amdgcn_readfirstlane(sh.next_tile);  // loaded during the previous tile
+            tb = p.tile_count[tile];
+        } else if (k == w) {
+            tile = first, tb = first_bin;
+        } else if constexpr (BATCH) {  // loaded during the previous tile
+            tile = __builtin_amdgcn_readfirstlane(sh.next_tile);
+            tb = TileBin{sh.next_count, sh.next_head};
         } else {
-            tile = k == w ? first : __builtin_amdgcn_readfirstlane(list[k]);
+            uint32_t lbase, lcap;
+            busy_list_span(p, xcd, lbase, lcap);
+            tile = __builtin_amdgcn_readfirstlane(p.busy[lbase + k]);
+            tb = p.tile_count[tile];
         }
-        TileBin tb = k == w && !nbig ? first_bin : TileBin{0u, 0u};
-        if (BATCH && k != w) tb = TileBin{sh.next_count, sh.next_head};
-        else if (k != w || nbig) tb = p.tile_count[tile];
         const uint32_t cnt = __builtin_amdgcn_readfirstlane(tb.count);
-        if (!(p.heavy_cap && cnt >= kHeavyTile)) {
-            run_tile(tile, cnt, __builtin_amdgcn_readfirstlane(tb.head), true);
-        } else {
-            if (tid == 0u) sh.next = per_xcd + atomicAdd(next, 1u);
+        if (heavy || !(p.heavy_cap && cnt >= kHeavyTile)) {
+            run_tile(tile, cnt, __builtin_amdgcn_readfirstlane(tb.head), !heavy);
+        } else {  // done already
+            __syncthreads();  // every lane has read sh.next
+            if (tid == 0u) sh.next = per_xcd + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
             __syncthreads();
         }
-        k = __builtin_amdgcn_readfirstlane(sh.next);
-        __syncthreads();
+        if (!heavy) k = __builtin_amdgcn_readfirstlane(sh.next);
     }
-    // 3. Empty tiles: groups of 8 consecutive tiles of the XCD's contiguous
-    //    range taken from its counter (the workgroups that finish their busy
-    //    tiles first take more of them), the clears, stores only.
+    // Empty tiles: groups of 8 consecutive tiles of the XCD's contiguous
+    // range taken from its counter (the workgroups that finish their busy
+    // tiles first take more of them), the clears, stores only.
+    const FrameParams &p = args();
     if ((BIG && nbig) || (!BATCH && !p.v0.clear_color_en && !p.v0.clear_depth_en)) return;
+    const uint32_t sx = p.tile_sx, sy = 8u - sx;
     uint32_t t0, t1;
-    xcd_range(ntiles, xcd, t0, t1);
-    uint32_t *empty = &p.ctr->empty[par][xcd][0];
+    xcd_range(p.ntiles, xcd, t0, t1);
+    uint32_t *empty = &p.ctr->empty[p.frame & 1u][xcd][0];
     for (;;) {
+        __syncthreads();  // sh.next has been read
         if (tid == 0u) sh.next = atomicAdd(empty, 8u);
         __syncthreads();
         const uint32_t base = t0 + __builtin_amdgcn_readfirstlane(sh.next);
-        __syncthreads();  // sh.next is written again next turn
         if (base >= t1) break;
         uint32_t c[8];
 #pragma unroll
@@ -1422,15 +1496,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(p.tile_req[tile]);
             const View &v = view_of<BATCH>(p, r);
             const uint32_t lt = tile - v.tile_base;
-            // one-sample kernels: the divisor made opaque here (an empty asm),
-            // so that its reciprocal is computed in this loop and not kept live
-            // through the whole kernel (where it took a register the shading needs)
-            uint32_t ntx = v.ntx;
-            if constexpr (!MS && !BIG) {
-                ntx = __builtin_amdgcn_readfirstlane(ntx);
-                asm volatile("" : "+s"(ntx));
-            }
-            const uint32_t ty = lt / ntx, tx = lt - ty * ntx;
+            const uint32_t ty = lt / v.ntx, tx = lt - ty * v.ntx;
             const uint32_t px = (tx << sx) + (tid & ((1u << sx) - 1u)), py = (ty << sy) + (tid >> sx);
             if (px < v.W && py < v.H) {
                 const size_t pidx = (size_t)py * v.W + px;
@@ -1713,8 +1779,7 @@ EUCHIP_DEV void span_item(const FrameParams &p, uint32_t b, void *static_lds) {
     // pixels the triangle covers (tile_bounds) raises its occluder bound.
     // Key order: Less + write takes zord, Greater + write ~zord; other depth
     // modes keep every entry (klo 0) and record no occluder.
-    const uint32_t mode = (p.depth_write && p.depth_test == DT_LESS) ? 1u
-                        : (p.depth_write && p.depth_test == DT_GREATER) ? 2u : 0u;
+    const uint32_t mode = key_mode(p);
     const uint32_t ty0 = ybase >> sy, all_rows = (1u << TH) - 1u;
     for (uint32_t i = lane; i < ne; i += 64u) {
         const uint32_t m = mb[i];
@@ -1859,8 +1924,7 @@ __global__ __launch_bounds__(256) void k_line_init(FrameParams p) {
     const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
     if (i >= (size_t)v.W * v.H) return;
     const bool uses_depth = p.depth_test != DT_NONE || p.depth_write;
-    const uint32_t mode = (p.depth_write && p.depth_test == DT_LESS) ? 1u
-                        : (p.depth_write && p.depth_test == DT_GREATER) ? 2u : 0u;
+    const uint32_t mode = key_mode(p);
     float D0 = 0.0f;
     if (uses_depth) D0 = v.clear_depth_en ? v.clear_depth : v.depth[i];
     p.lkey[i] = init_key(mode, D0);
@@ -1873,8 +1937,7 @@ __global__ __launch_bounds__(256) void k_line_raster(FrameParams p) {
     const View &v = p.v0;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6), nwaves = gridDim.x * 4u;
-    const uint32_t mode = (p.depth_write && p.depth_test == DT_LESS) ? 1u
-                        : (p.depth_write && p.depth_test == DT_GREATER) ? 2u : 0u;
+    const uint32_t mode = key_mode(p);
     for (uint32_t l = wave; l < p.n_lines; l += nwaves) {
         const uint4 *rq = reinterpret_cast<const uint4 *>(p.lrec + (size_t)l * kLineRecWords);
         const uint4 q0 = rq[0], q1 = rq[1], q2 = rq[2], q3 = rq[3];
@@ -1935,8 +1998,7 @@ __global__ __launch_bounds__(256) void k_line_resolve(FrameParams p) {
     const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
     if (i >= (size_t)v.W * v.H) return;
     const uint32_t px = (uint32_t)(i % v.W), py = (uint32_t)(i / v.W);
-    const uint32_t mode = (p.depth_write && p.depth_test == DT_LESS) ? 1u
-                        : (p.depth_write && p.depth_test == DT_GREATER) ? 2u : 0u;
+    const uint32_t mode = key_mode(p);
     const uint64_t kk = p.lkey[i];
     bool has;
     uint32_t prim;

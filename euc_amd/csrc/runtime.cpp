@@ -623,7 +623,7 @@ euchip_status render_impl(euchip_ctx *ctx, const euchip_pipeline_desc *d, const 
         if (ck_on) {
             p.ck_count = ctx->ck_count.ptr + par * half;
             if (ctx->ck_dirty[par])
-                HIP_TRY(ctx, launch_fill_u32((uint32_t *)p.ck_count, 0u, 2u * (size_t)ctx->ck_dirty[par], ctx->stream));
+                HIP_TRY(ctx, launch_fill_u32((uint32_t *)(uint2 *)p.ck_count, 0u, 2u * (size_t)ctx->ck_dirty[par], ctx->stream));
             ctx->ck_dirty[par] = 0;
         }
         p.ck_count_next = nullptr, p.ck_zero_n = 0u;
@@ -1281,6 +1281,7 @@ euchip_status euchip_render_noalloc(euchip_ctx *ctx, const euchip_pipeline_desc 
         return P.status;
     }
     uint8_t *base = static_cast<uint8_t *>(ctx->noalloc);
+    auto base_u32 = [&](size_t off) { return reinterpret_cast<uint32_t *>(base + off); };
     p.n_views = 1;
     p.ntiles = (uint32_t)ntiles;
     p.rec0 = reinterpret_cast<uint4 *>(base + kNaRec0);
@@ -1305,8 +1306,8 @@ euchip_status euchip_render_noalloc(euchip_ctx *ctx, const euchip_pipeline_desc 
     p.frame = 0;
     // the array keeps the last call's contents: counters and tile bins start at
     // zero (fill kernels: no memset nodes)
-    HIP_TRY(ctx, launch_fill_u32(reinterpret_cast<uint32_t *>(p.ctr), 0u, sizeof(Counters) / 4, st));
-    HIP_TRY(ctx, launch_fill_u32(reinterpret_cast<uint32_t *>(p.tile_count), 0u, 2 * ntiles, st));
+    HIP_TRY(ctx, launch_fill_u32(base_u32(kNaCtr), 0u, sizeof(Counters) / 4, st));
+    HIP_TRY(ctx, launch_fill_u32(base_u32(kNaTiles), 0u, 2 * ntiles, st));
     HIP_TRY(ctx, launch_setup(p, st, false, 0));
     HIP_TRY(ctx, launch_raster(p, st, false, ctx->max_groups));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->na_readback, &p.ctr->flags[0][0], 4, hipMemcpyDeviceToHost, st));
