@@ -1196,14 +1196,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
     const uint32_t tid = threadIdx.x;
     const uint32_t xcd = blockIdx.x & 7u;
     const uint32_t per_xcd = gridDim.x >> 3, w = blockIdx.x >> 3;
+    // Heavy tiles (the longest) go to the workgroups of the highest w, one each,
+    // and those own no busy tile: workgroup (w, xcd) takes heavy[hk], hk = 8 *
+    // (per_xcd - 1 - w) + xcd, then hk + gridDim.x, ...; the others take the busy
+    // tile w of their XCD's list first.
+    uint32_t hk = 8u * (per_xcd - 1u - w) + xcd;
     uint32_t nh, nbusy, nbig, first, pool_used;
     TileBin first_bin;
     {
         const FrameParams &p = args();
         const uint32_t par = p.frame & 1u, npar = (p.frame + 1u) & 1u;
         // The loads the first tile waits for, issued together: frame flags, pool use,
-        // list lengths, this workgroup's first busy tile and its bin state (read at a
-        // clamped index before the tile is known to be in the list; used only if it is).
+        // list lengths, this workgroup's first tile in either list and its bin state
+        // (read at a clamped index before the tile is known to be in the list; used
+        // only if it is).
         uint32_t lbase, lcap;
         busy_list_span(p, xcd, lbase, lcap);
         const uint32_t flags = p.ctr->flags[par][0];
@@ -1212,7 +1218,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         // big triangles (with checkpoints any triangle may be on any tile's list)
         nbig = !BIG ? 0u : p.ck_on ? p.v0.n_tris : __builtin_amdgcn_readfirstlane(p.ctr->big[par][0]);
         nbusy = __builtin_amdgcn_readfirstlane(p.ctr->busy[par][xcd][0]);
-        first = w < lcap ? __builtin_amdgcn_readfirstlane(p.busy[lbase + w]) : 0u;
+        const uint32_t first_busy = w < lcap ? __builtin_amdgcn_readfirstlane(p.busy[lbase + w]) : 0u;
+        const uint32_t first_heavy = hk < p.heavy_cap ? __builtin_amdgcn_readfirstlane(p.heavy[hk]) : 0u;
+        nh = nh < p.heavy_cap ? nh : p.heavy_cap;
+        first = hk < nh ? first_heavy : first_busy;
         first_bin = p.tile_count[first < p.ntiles ? first : 0u];
         if (p.report && blockIdx.x == 0u && tid == 0u) {
             // this frame's setup counts, for the host (frame number last)
@@ -1253,9 +1262,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             xcd_range(p.ntiles, xcd, b0, b1);
             nbusy = b1 - b0;
         }
-        nh = nh < p.heavy_cap ? nh : p.heavy_cap;
         nbusy = nbusy < lcap ? nbusy : lcap;
     }
+    // where this XCD's counter starts: the busy tiles that its workgroups do not own
+    const uint32_t hx = nh > xcd ? (nh - xcd + 7u) >> 3 : 0u;  // its workgroups that take a heavy tile (and more: a second)
+    const uint32_t owned = hx < per_xcd ? per_xcd - hx : 0u;
 
     // One tile with `cnt` bin entries and overflow list `head`: winner keys in
     // LDS, then the resolve.
@@ -1274,7 +1285,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         bool ckp = false;  // big triangles from their row checkpoints (else walked from the row starts)
         {
             const FrameParams &p = args();
-            if (BATCH && claim && tid == 0u) claimed = per_xcd + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
+            if (BATCH && claim && tid == 0u) claimed = owned + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
             if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(p.tile_req[tile]);
             const View &v = view_of<BATCH>(p, r);
             lt = tile - v.tile_base;
@@ -1367,7 +1378,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
                 ntile = p.busy[lbase + claimed];
                 ntb = p.tile_count[ntile];
             }
-            if (!BATCH && claim && tid == 0u) claimed = per_xcd + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
+            if (!BATCH && claim && tid == 0u) claimed = owned + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
             const uint32_t px = g.X0 + (tid & (g.TW - 1u)), py = g.Y0 + (tid >> sx);
             if (px < v.W && py < v.H) {
                 const size_t pidx = (size_t)py * v.W + px;
@@ -1427,26 +1438,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         __syncthreads();
     };
 
-    // Heavy tiles first, workgroup k taking heavy[k] (the longest tiles start
-    // early instead of ending the launch late); then the busy tiles of this XCD's
-    // list: the first by workgroup index, the rest from the XCD's counter (heavy
-    // ones are done).  One loop, so one copy of the tile code.
-    for (uint32_t hk = blockIdx.x, k = w;;) {
+    // This workgroup's heavy tiles (so that the longest tiles start early instead
+    // of ending the launch late), or its own busy tile, then busy tiles from the
+    // XCD's counter (the heavy ones among them are done).  One loop, so one copy
+    // of the tile code.
+    for (uint32_t k = hk < nh ? ~0u : w, round = 0u;; round++) {
         const bool heavy = hk < nh;
         if (!heavy && k >= nbusy) break;
         const FrameParams &p = args();
         uint32_t tile;
         TileBin tb;
-        if (heavy) {
-            tile = __builtin_amdgcn_readfirstlane(p.heavy[hk]);
-            tb = p.tile_count[tile];
-            hk += gridDim.x;
-        } else if (BIG && nbig) {
+        if (BIG && nbig && !heavy) {
             uint32_t b0, b1;
             xcd_range(p.ntiles, xcd, b0, b1);
             tile = b0 + k;
             tb = p.tile_count[tile];
-        } else if (k == w) {
+        } else if (round == 0u) {
             tile = first, tb = first_bin;
         } else if constexpr (BATCH) {  // loaded during the previous tile
             tile = __builtin_amdgcn_readfirstlane(sh.next_tile);
@@ -1454,18 +1461,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         } else {
             uint32_t lbase, lcap;
             busy_list_span(p, xcd, lbase, lcap);
-            tile = __builtin_amdgcn_readfirstlane(p.busy[lbase + k]);
+            tile = __builtin_amdgcn_readfirstlane(heavy ? p.heavy[hk] : p.busy[lbase + k]);
             tb = p.tile_count[tile];
         }
+        if (heavy) hk += gridDim.x;
+        const bool claim = hk >= nh;  // the next tile comes from the counter
         const uint32_t cnt = __builtin_amdgcn_readfirstlane(tb.count);
         if (heavy || !(p.heavy_cap && cnt >= kHeavyTile)) {
-            run_tile(tile, cnt, __builtin_amdgcn_readfirstlane(tb.head), !heavy);
+            run_tile(tile, cnt, __builtin_amdgcn_readfirstlane(tb.head), claim);
         } else {  // done already
             __syncthreads();  // every lane has read sh.next
-            if (tid == 0u) sh.next = per_xcd + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
+            if (tid == 0u) sh.next = owned + atomicAdd(&p.ctr->next[p.frame & 1u][xcd][0], 1u);
             __syncthreads();
         }
-        if (!heavy) k = __builtin_amdgcn_readfirstlane(sh.next);
+        if (claim) k = __builtin_amdgcn_readfirstlane(sh.next);
     }
     // Empty tiles: groups of 8 consecutive tiles of the XCD's contiguous
     // range taken from its counter (the workgroups that finish their busy
