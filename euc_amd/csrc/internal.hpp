@@ -75,8 +75,6 @@ enum FrameFlags : uint32_t { FLAG_BIN_OVERFLOW = 1u };
 // 128-byte line.
 struct Counters {
     uint32_t pool[2][32];     // words of the overflow pool taken
-    uint32_t next[2][8][32];  // per XCD: next tile of the dynamic tile loop
-    uint32_t empty[2][8][32]; // per XCD: next group of tiles the empty-tile clears look at
     uint32_t heavy[2][32];    // entries of the heavy-tile list
     uint32_t big[2][32];      // entries of the big-triangle list
     uint32_t busy[2][8][32];  // per XCD: entries of the busy-tile list
@@ -226,6 +224,7 @@ struct FrameParams {
     gptr<Report> report;        // host-visible report of one-request frames, or null
     gptr<uint32_t> heavy;       // tiles with at least kHeavyTile entries (heavy_cap slots)
     uint32_t heavy_cap;    // 0: no heavy-first pass
+    uint32_t heavy_groups; // raster workgroups that take the heavy tiles, a multiple of 8
     // Setup lists the tiles it bins into (busy) in 8 lists of up to ntiles
     // entries (list x at busy + x * ntiles, chosen by busy_map); raster clears
     // the empty tiles itself, takes only busy tiles from the lists, leaves
@@ -296,7 +295,7 @@ hipError_t noalloc_scratch(int device, void **out);
 // kernels that read their requests from p.views (setup then runs `blocks`
 // workgroups as p.blk maps them); one-request launches read p.v0.
 hipError_t launch_setup(const FrameParams &p, hipStream_t s, bool batched, uint32_t blocks);
-hipError_t launch_raster(const FrameParams &p, hipStream_t s, bool batched, uint32_t max_groups);
+hipError_t launch_raster(const FrameParams &p, hipStream_t s, bool batched);
 // Row checkpoints of the big triangles (one-request big-triangle frames with a
 // checkpoint pool), between setup and raster.
 hipError_t launch_fill_u32(uint32_t *dst, uint32_t value, size_t n, hipStream_t s);

@@ -80,7 +80,6 @@ struct euchip_ctx {
     uint32_t tile_cap = 128;    // bin slots per tile; raised when a frame needed more (within the bin budget)
     size_t pool_want = 0;       // pool words the next frames should have (from the reports)
     uint32_t frame = 0;
-    uint32_t max_groups = 2048; // resident raster workgroups: CUs x 8
     uint32_t big_tile_sx = 5;   // tiles of big-triangle frames: (1 << sx) x (256 >> sx) pixels
     Counters *counters = nullptr;
     Report *report = nullptr;   // host memory the raster pass writes each frame's counts to
@@ -651,7 +650,7 @@ euchip_status render_impl(euchip_ctx *ctx, const euchip_pipeline_desc *d, const 
         p.heavy_cap = (uint32_t)std::min<size_t>(ctx->heavy.cap, 0xFFFFFFF0ull);
         p.frame = ctx->frame++;
         if ((s = timed(ctx, "setup", [&] { return launch_setup(p, ctx->stream, false, 0); }))) return s;
-        if ((s = timed(ctx, "raster", [&] { return launch_raster(p, ctx->stream, false, ctx->max_groups); }))) return s;
+        if ((s = timed(ctx, "raster", [&] { return launch_raster(p, ctx->stream, false); }))) return s;
         ctx->counts_used[npar] = 0;
         ctx->counts_used[par] = (uint32_t)ntiles;
         if (p.ck_zero_n) ctx->ck_dirty[npar] = 0;
@@ -846,11 +845,11 @@ euchip_status enqueue_batch(euchip_batch *b, bool capturing = false) {
     if (ctx->profiling && !capturing) {
         if ((s = timed_on(ctx, b->stream, "batch_setup", [&] { return launch_setup(b->p, b->stream, true, b->setup_blocks); })))
             return s;
-        if ((s = timed_on(ctx, b->stream, "batch_raster", [&] { return launch_raster(b->p, b->stream, true, ctx->max_groups); })))
+        if ((s = timed_on(ctx, b->stream, "batch_raster", [&] { return launch_raster(b->p, b->stream, true); })))
             return s;
     } else {
         HIP_TRY(ctx, launch_setup(b->p, b->stream, true, b->setup_blocks));
-        HIP_TRY(ctx, launch_raster(b->p, b->stream, true, ctx->max_groups));
+        HIP_TRY(ctx, launch_raster(b->p, b->stream, true));
     }
     HIP_TRY(ctx, hipMemcpyAsync(b->host_ctr, b->ctrbuf.ptr, words * 4, hipMemcpyDeviceToHost, b->stream));
     return EUCHIP_OK;
@@ -988,9 +987,6 @@ euchip_status euchip_ctx_create(int device, euchip_ctx **out) {
         const int v = atoi(e);
         if (v >= 3 && v <= 8) ctx->big_tile_sx = (uint32_t)v;
     }
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0)
-        ctx->max_groups = (uint32_t)cus * 8u;
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc((void **)&ctx->counters, sizeof(Counters)) != hipSuccess ||
         hipHostMalloc((void **)&ctx->report, sizeof(Report), hipHostMallocDefault) != hipSuccess ||
@@ -1309,7 +1305,7 @@ euchip_status euchip_render_noalloc(euchip_ctx *ctx, const euchip_pipeline_desc 
     HIP_TRY(ctx, launch_fill_u32(base_u32(kNaCtr), 0u, sizeof(Counters) / 4, st));
     HIP_TRY(ctx, launch_fill_u32(base_u32(kNaTiles), 0u, 2 * ntiles, st));
     HIP_TRY(ctx, launch_setup(p, st, false, 0));
-    HIP_TRY(ctx, launch_raster(p, st, false, ctx->max_groups));
+    HIP_TRY(ctx, launch_raster(p, st, false));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->na_readback, &p.ctr->flags[0][0], 4, hipMemcpyDeviceToHost, st));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->na_readback + 1, &p.ctr->pool[0][0], 4, hipMemcpyDeviceToHost, st));
     HIP_TRY(ctx, hipStreamSynchronize(st));

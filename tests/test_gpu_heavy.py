@@ -32,6 +32,7 @@ def scattered(seed, n, extent, size, n_large=0):
     (250, 190, 6000, 0.3, 0.02, 0),        # some heavy
     (640, 480, 3000, 1.0, 0.004, 0),       # none heavy, some empty
     (1024, 800, 600000, 1.0, 0.004, 0),    # 3200 tiles, most heavy: more than the workgroups
+    (3000, 1800, 20000, 1.0, 0.01, 0),     # 21,150 tiles: several per workgroup
     (2048, 2048, 1000, 0.01, 0.01, 8),     # big-triangle frame without checkpoints, a few heavy tiles
 ])
 def test_heavy_tiles(gpu_ctx, w, h, n, extent, size, n_large):
