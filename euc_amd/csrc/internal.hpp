@@ -241,7 +241,8 @@ struct FrameParams {
     // halves by frame parity like tile_count: ck_count this frame's,
     // ck_count_next the other, whose first ck_zero_n counts a big-triangle
     // frame's raster zeroes).
-    // A one-request setup launch has tri_blocks triangle blocks, then vertex
+    // A one-request setup launch has tri_blocks blocks of tri_block triangles
+    // each, then vertex
     // blocks up to setup_blocks; a checkpoint frame's has setup_blocks blocks
     // of triangles and vertices, then the span blocks (span_parts items of
     // kSpanRows rows per triangle, 4 per block).
@@ -252,7 +253,7 @@ struct FrameParams {
     uint32_t mstride;
     gptr<uint2> ck_count, ck_count_next;  // per tile (list length, ~least occluder bound)
     uint32_t ck_zero_n;
-    uint32_t tri_blocks, setup_blocks, span_parts;
+    uint32_t tri_block, tri_blocks, setup_blocks, span_parts;
     gptr<TileBin> count_next;
     uint32_t zero_n;
     uint32_t frame;        // frame parity selects the overflow counter and tile queue
