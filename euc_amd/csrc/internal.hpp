@@ -159,6 +159,33 @@ constexpr uint32_t span_table_bytes(uint32_t sy, uint32_t ntx) {
 constexpr uint32_t kBigRecQuads = 2;
 constexpr size_t kCkMaxSlots = (size_t)1 << 26;  // 1 GiB of checkpoints at most
 
+// A divisor d >= 1 of 32-bit numbers fixed when a launch is prepared: n / d by a
+// high multiply and shifts (Granlund and Montgomery 1994, figure 4.1), exact for
+// every n.  A 32-bit division by a value known only in the kernel takes about
+// twenty vector instructions, also where both operands are uniform.
+struct Divisor {
+    uint32_t d, mul, shift1, shift2;
+};
+inline Divisor make_divisor(uint32_t d) {
+    uint32_t l = 0;
+    while (l < 32 && ((uint64_t)1 << l) < d) l++;
+    const uint64_t mul = ((((uint64_t)1 << l) - d) << 32) / d + 1;
+    return Divisor{d, (uint32_t)mul, l < 1 ? l : 1u, l < 1 ? 0u : l - 1u};
+}
+__host__ __device__ inline uint32_t divide(uint32_t n, const Divisor &v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint32_t t = __umulhi(v.mul, n);
+#else
+    const uint32_t t = (uint32_t)(((uint64_t)v.mul * n) >> 32);
+#endif
+    return (t + ((n - t) >> v.shift1)) >> v.shift2;
+}
+
+// How a primitive's corners map to instances: every instance holds whole
+// triangles (instance t / tris.d), there is one instance, or neither (a trailing
+// partial triangle continues in the next instance: each corner is divided apart).
+enum InstanceMap : uint32_t { INST_CORNERS = 0, INST_TRIANGLES = 1, INST_ONE = 2 };
+
 // One render request: a target pair, a mesh, a uniform block, and where the
 // request's vertices, tiles and bins sit in the launch's scratch memory.
 struct View {
@@ -185,6 +212,10 @@ struct View {
     gptr<const uint32_t> idx;
     gptr<const float> models;
     uint32_t pos_comps, count, n_vertices, n_instances, n_tris;
+    uint32_t inst_map;     // InstanceMap
+    Divisor inst_tris;     // triangles per instance (INST_TRIANGLES)
+    Divisor inst_verts;    // vertices per instance
+    Divisor row_tiles;     // ntx
     // textures (device)
     gptr<const uint32_t> tex;
     uint32_t tex_w, tex_h;

@@ -44,7 +44,6 @@ EUCHIP_DEV uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_
 // registers went to vector-register lanes, and every use of it took a
 // v_readlane: a quarter of the raster kernels' vector instructions).  Scalar
 // loads of a line that the scalar cache holds cost no vector issue at all.
-#define EUCHIP_CONST __attribute__((address_space(4)))
 EUCHIP_DEV const FrameParams &args() {
     const EUCHIP_CONST FrameParams *k = (const EUCHIP_CONST FrameParams *)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(k));
@@ -95,6 +94,21 @@ EUCHIP_DEV uint32_t corner_element(uint32_t geometry, uint32_t t, int i) {
     return 3u * tri + c;
 }
 
+// Instance and index within the instance of the corners of primitive t.
+EUCHIP_DEV void corner_places(const View &v, uint32_t geometry, uint32_t t, uint32_t inst[3], uint32_t at[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) inst[i] = 0u, at[i] = corner_element(geometry, t, i);
+    if (v.inst_map == INST_TRIANGLES) {
+        const uint32_t tri = geometry == GEOM_BOTH_SIDES ? t >> 1 : t;
+        const uint32_t q = divide(tri, v.inst_tris);
+#pragma unroll
+        for (int i = 0; i < 3; i++) inst[i] = q, at[i] -= q * v.count;
+    } else if (v.inst_map == INST_CORNERS) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) inst[i] = at[i] / v.count, at[i] -= inst[i] * v.count;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // triangle setup (triangles.rs:55-171) of primitive t of request v, whole-target
 // band clamp, from the vertex shader's clip positions.  Returns false when the
@@ -107,12 +121,7 @@ EUCHIP_DEV bool tri_setup(const FrameParams &p, const View &v, uint32_t t, TriRe
     // the corners' clip positions (vertex(): VP * model * (p, 1), or the CLIP
     // input itself), the uniform branches taken outside the corner loop so the
     // loads of all three corners are in flight together
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const uint32_t e = corner_element(p.geometry, t, i);
-        inst[i] = e / v.count;
-        vi[i] = e - inst[i] * v.count;
-    }
+    corner_places(v, p.geometry, t, inst, vi);
     if (v.idx) {
 #pragma unroll
         for (int i = 0; i < 3; i++) vi[i] = v.idx[vi[i]];
@@ -133,14 +142,23 @@ EUCHIP_DEV bool tri_setup(const FrameParams &p, const View &v, uint32_t t, TriRe
             }
         }
     } else {
+        float p4[3][4], w[3][4];
 #pragma unroll
         for (int i = 0; i < 3; i++) {
             const float *P = v.pos + (size_t)v.pos_comps * vi[i];
-            const float p4[4] = {P[0], P[1], P[2], 1.0f};
-            float w[4];
-            mat4_vec4(v.models + 16u * inst[i], p4, w);
-            mat4_vec4(v.u + U_VP, w, c[i]);
+            p4[i][0] = P[0], p4[i][1] = P[1], p4[i][2] = P[2], p4[i][3] = 1.0f;
         }
+        if (v.inst_map == INST_CORNERS) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) mat4_vec4((const float *)v.models + 16u * inst[i], p4[i], w[i]);
+        } else {
+            with_model(v, inst[0], [&](const EUCHIP_CONST float *m) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) mat4_vec4(m, p4[i], w[i]);
+            });
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++) mat4_vec4(v.u + U_VP, w[i], c[i]);
     }
 #pragma unroll
     for (int i = 0; i < 3; i++) {
@@ -296,7 +314,7 @@ EUCHIP_DEV void busy_list_span(const FrameParams &p, uint32_t x, uint32_t &base,
 // Busy list of a tile.
 EUCHIP_DEV uint32_t busy_list_of(const FrameParams &p, uint32_t tile) {
     if (p.busy_map == BUSY_BLOCKS) {  // one request: blocks of 4 x 4 tiles dealt over the XCDs
-        const uint32_t ty = tile / p.v0.ntx, tx = tile - ty * p.v0.ntx;
+        const uint32_t ty = divide(tile, p.v0.row_tiles), tx = tile - ty * p.v0.ntx;
         return ((tx >> 2) + 3u * (ty >> 2)) & 7u;
     }
     // the XCD whose contiguous tile range (xcd_range) holds the tile
@@ -413,13 +431,14 @@ EUCHIP_DEV void load_rec1(const FrameParams &p, uint32_t rid, TriRec &R) {
 
 // Shaded-vertex ids of primitive t's corners after the winding swap.
 EUCHIP_DEV void tri_sids(const View &v, uint32_t geometry, uint32_t t, uint32_t flags, uint32_t sid[3]) {
+    uint32_t inst[3], at[3];
+    corner_places(v, geometry, t, inst, at);
+    if (v.idx) {
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const uint32_t e = corner_element(geometry, t, i);
-        const uint32_t inst = e / v.count;
-        const uint32_t k = e - inst * v.count;
-        sid[i] = v.sv_base + inst * v.n_vertices + (v.idx ? v.idx[k] : k);
+        for (int i = 0; i < 3; i++) at[i] = v.idx[at[i]];
     }
+#pragma unroll
+    for (int i = 0; i < 3; i++) sid[i] = v.sv_base + inst[i] * v.n_vertices + at[i];
     if (flags & TRI_SWAPPED) {
         const uint32_t s0 = sid[0];
         sid[0] = sid[2];
@@ -521,7 +540,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
                 const View &v = p.v0;
                 const uint32_t t = (blockIdx.x - p.tri_blocks) * 256u + tid;
                 if (t < v.n_instances * v.n_vertices) {
-                    const uint32_t inst = t / v.n_vertices;
+                    const uint32_t inst = divide(t, v.inst_verts);
                     float vd[VDN<SH>::N];
                     vertex_data<SH>(p, v, inst, t - inst * v.n_vertices, vd);
 #pragma unroll
@@ -583,7 +602,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     // other one-request frames have vertex blocks of their own.
     if constexpr ((BATCH || SPAN) && vd_count(SH) > 0) {  // (their workgroups have 256 triangles)
         if (t < v.n_instances * v.n_vertices) {
-            const uint32_t inst = t / v.n_vertices;
+            const uint32_t inst = divide(t, v.inst_verts);
             const uint32_t vi = t - inst * v.n_vertices;
             const size_t sv = (size_t)v.sv_base + t;
             float vd[VDN<SH>::N];
@@ -1310,7 +1329,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(uniform_load(p.tile_req + tile));
             const View &v = view_of<BATCH>(p, r);
             lt = tile - v.tile_base;
-            const uint32_t ty = lt / v.ntx, tx = lt - ty * v.ntx;
+            const uint32_t ty = divide(lt, v.row_tiles), tx = lt - ty * v.ntx;
             sx = p.tile_sx;
             g.sx = sx, g.TW = 1u << sx, g.TH = 256u >> sx;
             g.X0 = tx << sx, g.Y0 = ty << (8u - sx);
@@ -1486,7 +1505,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(uniform_load(p.tile_req + tile));
             const View &v = view_of<BATCH>(p, r);
             const uint32_t lt = tile - v.tile_base;
-            const uint32_t ty = lt / v.ntx, tx = lt - ty * v.ntx;
+            const uint32_t ty = divide(lt, v.row_tiles), tx = lt - ty * v.ntx;
             const uint32_t px = (tx << sx) + (tid & ((1u << sx) - 1u)), py = (ty << (8u - sx)) + (tid >> sx);
             if (px < v.W && py < v.H) {
                 const size_t pidx = (size_t)py * v.W + px;
@@ -1816,7 +1835,7 @@ EUCHIP_DEV void element_clip(const FrameParams &p, const View &v, uint32_t e, fl
     } else {
         const float p4[4] = {P[0], P[1], P[2], 1.0f};
         float w[4];
-        mat4_vec4(v.models + 16u * inst, p4, w);
+        mat4_vec4((const float *)v.models + 16u * inst, p4, w);
         mat4_vec4(v.u + U_VP, w, c);
     }
     sid = v.sv_base + inst * v.n_vertices + vi;
@@ -1850,7 +1869,7 @@ __global__ __launch_bounds__(256) void k_line_setup(FrameParams p) {
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     if constexpr (vd_count(SH) > 0) {
         if (t < v.n_instances * v.n_vertices) {
-            const uint32_t inst = t / v.n_vertices;
+            const uint32_t inst = divide(t, v.inst_verts);
             float vd[VDN<SH>::N];
             vertex_data<SH>(p, v, inst, t - inst * v.n_vertices, vd);
 #pragma unroll

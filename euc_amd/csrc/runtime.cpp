@@ -445,6 +445,9 @@ euchip_status plan_request(euchip_ctx *ctx, const euchip_pipeline_desc *d, const
     v.idx = mesh->idx, v.models = mesh->models;
     v.pos_comps = mesh->pos_comps, v.count = mesh->count, v.n_vertices = mesh->n_vertices;
     v.n_instances = mesh->n_instances, v.n_tris = (uint32_t)P.n_tris;
+    v.inst_map = mesh->n_instances == 1 ? INST_ONE : mesh->count % 3 == 0 ? INST_TRIANGLES : INST_CORNERS;
+    v.inst_tris = make_divisor(std::max<uint32_t>(mesh->count / 3, 1u));
+    v.inst_verts = make_divisor(std::max<uint32_t>(mesh->n_vertices, 1u));
     if (texture) v.tex = (const uint32_t *)texture->ptr, v.tex_w = texture->w, v.tex_h = texture->h;
     if (shadow) v.shadow = (const float *)shadow->ptr, v.sh_w = shadow->w, v.sh_h = shadow->h;
     memcpy(v.u, uniforms, sizeof(v.u));
@@ -456,6 +459,7 @@ void tile_grid(View &v, uint32_t sx) {
     const uint32_t tw = 1u << sx, th = 256u >> sx;
     v.ntx = (v.W + tw - 1) / tw;
     v.nty = (v.H + th - 1) / th;
+    v.row_tiles = make_divisor(std::max<uint32_t>(v.ntx, 1u));
 }
 
 euchip_status enqueue_clears(euchip_ctx *ctx, const euchip_pipeline_desc *d, const Plan &P, euchip_buffer *pixel,

@@ -41,7 +41,8 @@ EUCHIP_DEV uint32_t sat_u8(float f) {
     return (uint32_t)f;
 }
 
-EUCHIP_DEV void mat4_vec4(const float *m, const float v[4], float r[4]) {
+template <class M>  // a matrix in any memory
+EUCHIP_DEV void mat4_vec4(const M *m, const float v[4], float r[4]) {
 #pragma unroll
     for (int i = 0; i < 4; i++)
         r[i] = ((m[4 * i + 0] * v[0] + m[4 * i + 1] * v[1]) + m[4 * i + 2] * v[2]) + m[4 * i + 3] * v[3];
@@ -170,15 +171,43 @@ EUCHIP_DEV void sample_rgba8(const uint32_t *tex, uint32_t w, uint32_t h, uint32
 // Pipeline::vertex of the fixed shader set
 // ---------------------------------------------------------------------------
 
-// World position (model * (p, 1)) or, for CLIP input, the position itself.
-EUCHIP_DEV void vertex_world(const FrameParams &p, const View &v, uint32_t inst, uint32_t vi, float wpos[4]) {
+// f(model matrix of instance inst): the matrix is read by scalar loads, for one
+// instance of the wave's lanes after the other (nearly always there is one only;
+// a lane's own copy took 4 vector loads of 16 bytes each).  No kernel writes
+// the matrices.
+#define EUCHIP_CONST __attribute__((address_space(4)))
+template <class F>
+EUCHIP_DEV void with_model(const View &v, uint32_t inst, F f) {
+    const EUCHIP_CONST float *models = (const EUCHIP_CONST float *)(const float *)v.models;
+    if (v.inst_map == INST_ONE) {
+        f(models);
+        return;
+    }
+    for (bool done = false; !done;) {
+        const uint32_t u = __builtin_amdgcn_readfirstlane(inst);
+        if (inst == u) {
+            f(models + 16u * (size_t)u);
+            done = true;
+        }
+    }
+}
+
+// World position (model * (p, 1)) or, for CLIP input, the position itself, and
+// the normal through the model (or as it is).
+EUCHIP_DEV void vertex_world(const FrameParams &p, const View &v, uint32_t inst, uint32_t vi, const float n4[4],
+                             float wpos[4], float wn[4]) {
     const float *P = v.pos + (size_t)v.pos_comps * vi;
     if (p.xform == 0) {
         wpos[0] = P[0], wpos[1] = P[1], wpos[2] = P[2];
         wpos[3] = v.pos_comps == 4 ? P[3] : 1.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) wn[i] = n4[i];
     } else {
         const float p4[4] = {P[0], P[1], P[2], 1.0f};
-        mat4_vec4(v.models + 16u * inst, p4, wpos);
+        with_model(v, inst, [&](const EUCHIP_CONST float *m) {
+            mat4_vec4(m, p4, wpos);
+            mat4_vec4(m, n4, wn);
+        });
     }
 }
 
@@ -196,12 +225,10 @@ EUCHIP_DEV void vertex_data(const FrameParams &p, const View &v, uint32_t inst, 
         (void)vd;
     } else {
         float wpos[4], wn[4];
-        vertex_world(p, v, inst, vi, wpos);
         const float *N = v.nrm + 3u * vi;
         float n4[4] = {N[0], N[1], N[2], 0.0f};
         if constexpr (SH == PHONG_SHADOW) n4[0] = -N[0], n4[1] = -N[1], n4[2] = -N[2];
-        if (p.xform == 0) wn[0] = n4[0], wn[1] = n4[1], wn[2] = n4[2], wn[3] = n4[3];
-        else mat4_vec4(v.models + 16u * inst, n4, wn);
+        vertex_world(p, v, inst, vi, n4, wpos, wn);
         if constexpr (SH == GOURAUD) {
             lighting2(v.u, wpos, wn, vd);
         } else {
