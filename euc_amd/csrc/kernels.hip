@@ -1320,6 +1320,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
     auto run_tile = [&](uint32_t tile, uint32_t cnt, uint32_t head, uint32_t ntile, TileBin &ntb) {
         uint32_t r = 0u, lt, sx, nck = 0u, occl = 0u, run, nb, tri_base;
         uint64_t bin_at;  // first bin slot of the tile
+        uint32_t ahead = 0u;  // this lane's entry of the next step of the bin, loaded a step ahead
         uint32_t seg = 0u;
         TileGeom g;
         uint2 e_first = make_uint2(0u, 0u);
@@ -1329,6 +1330,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(uniform_load(p.tile_req + tile));
             const View &v = view_of<BATCH>(p, r);
             lt = tile - v.tile_base;
+            tri_base = v.tri_base;
+            bin_at = v.bin_base + (uint64_t)lt * v.tile_cap;
+            nb = cnt < v.tile_cap ? cnt : v.tile_cap;
+            seg = cnt > v.tile_cap ? head : 0u;
+            if (tid < kBatch && tid < nb) ahead = p.bins[bin_at + tid];
             const uint32_t ty = divide(lt, v.row_tiles), tx = lt - ty * v.ntx;
             sx = p.tile_sx;
             g.sx = sx, g.TW = 1u << sx, g.TH = 256u >> sx;
@@ -1348,11 +1354,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
                 sh.band[2 * tid] = by0;
                 sh.band[2 * tid + 1] = by1;
             }
-            const uint32_t cap = v.tile_cap;
-            tri_base = v.tri_base;
-            bin_at = v.bin_base + (uint64_t)lt * cap;
-            nb = cnt < cap ? cnt : cap;
-            seg = cnt > cap ? head : 0u;
             // the tile's checkpoint list: its length and first 256 entries, loaded
             // now (used after the bin; entries past the length are ignored)
             if constexpr (BIG) {
@@ -1397,7 +1398,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
                 // (read once; a plain load would be merged with the bin's into one FLAT load)
                 valid = true, prim = __builtin_nontemporal_load(&args().pool[base + i]);
             } else if (i < nb) {
-                valid = true, prim = args().bins[bin_at + i];
+                valid = true, prim = ahead;
+                if (i + kBatch < nb) ahead = args().bins[bin_at + i + kBatch];
             } else if constexpr (BIG) {
                 valid = true, prim = args().big[i - nb];
             }
