@@ -935,7 +935,8 @@ EUCHIP_DEV void walk_row(const FrameParams &p, const TriRec &R, uint32_t prim, u
     }
 }
 
-// The write modes' row loop: coverage, z, z clip and the key of every pixel,
+// The row loop of the write modes and of frames without a depth test: coverage,
+// z, z clip and the key of every pixel,
 // then one LDS atomic min per pixel, with no branch: an uncovered pixel's
 // atomic takes the all-ones key, which changes nothing.  The loop holds no LDS
 // read, so nothing waits on the atomics of earlier pixels.
@@ -947,6 +948,11 @@ EUCHIP_DEV void walk_row(const FrameParams &p, const TriRec &R, uint32_t prim, u
 //     z ^ (z + 0) shifted in beside (prim + 1) keeps the sign in the key.
 //   * An uncovered pixel's key has an all-ones high word: no stored key has
 //     one (order values of non-NaN depths stay below it), so it never wins.
+//   * MODE 3 (no depth test, no such write): the last fragment wins whatever its
+//     z, a NaN among them, so the weights are tested one by one and an uncovered
+//     pixel's atomic max takes zero, which changes nothing either.  (Reading the
+//     depth before the pass for a test that always passes, with its atomic under
+//     a branch, took 9 us for a tile's rows of 32 pixels.)
 //   * PAIRS: two pixels per turn (the second atomic at the next address)
 //     halve the loop control; a row of odd length ends with one more pixel.
 //     It pays for long rows only.
@@ -956,9 +962,18 @@ EUCHIP_DEV void walk_keys(const TriRec &R, bool clip, float zlo, float zhi, uint
     auto pixel = [&](unsigned long long *at) {
         const float u2 = (w2 - w0) - w1;
         const float z = (R.hz[0] * w0 + R.hz[1] * w1) + R.hz[2] * u2;
-        bool ok = (__builtin_fminf(__builtin_fminf(w0, w1), u2) >= 0.0f) & (z == z);
+        bool ok;
+        if constexpr (MODE == 3u) ok = (w0 >= 0.0f) & (w1 >= 0.0f) & (u2 >= 0.0f);
+        else ok = (__builtin_fminf(__builtin_fminf(w0, w1), u2) >= 0.0f) & (z == z);
         if constexpr (CLIP) ok = ok & (!clip | ((zlo <= z) & (z <= zhi)));
         const uint32_t bz = __float_as_uint(z), u = __float_as_uint(z + 0.0f);
+        if constexpr (MODE == 3u) {
+            atomicMax(at, ok ? ((uint64_t)pid << 32) | bz : 0ull);
+            w0 = w0 + R.dx[0];
+            w1 = w1 + R.dx[1];
+            w2 = w2 + R.dx[2];
+            return;
+        }
         const uint32_t o = u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
         const uint32_t lo = __builtin_amdgcn_alignbit(pid, bz ^ u, 31u);  // (pid << 1) | (z is -0)
         const uint32_t hi = ok ? (MODE == 1u ? o : ~o) : ~0u;
@@ -980,8 +995,8 @@ EUCHIP_DEV void walk_keys(const TriRec &R, bool clip, float zlo, float zhi, uint
     }
 }
 
-// walk_row without branches on the coverage; the write modes take walk_keys,
-// with the z clip only where a lane of the wave needs it.
+// walk_row without branches on the coverage; the write modes and frames without
+// a depth test take walk_keys, with the z clip only where a lane of the wave needs it.
 template <uint32_t MODE, bool PAIRS = false>
 EUCHIP_DEV void walk_span(const FrameParams &p, const TriRec &R, uint32_t prim, uint32_t xs, uint32_t xe, uint32_t pi0,
                           float w0, float w1, float w2, uint64_t *key, const float *d0s) {
@@ -1049,6 +1064,7 @@ EUCHIP_DEV void raster_row(const FrameParams &p, const TriRec &R, uint32_t prim,
     // the long-row variant (big-triangle kernels) walks two pixels per turn
     if (mode == 1u) walk_span<1u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
     else if (mode == 2u) walk_span<2u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
+    else if (p.depth_test == DT_NONE) walk_span<3u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
     else walk_row<0u>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
 }
 
@@ -1218,6 +1234,7 @@ EUCHIP_DEV void big_tasks(const FrameParams &p, TileShared &sh, uint32_t tid, ui
                 const float w2 = __uint_as_float(c[h].z);
                 if (mode == 1u) walk_span<1u, true>(p, R, x6[h].x, xs, xe, pi0, w0, w1, w2, sh.key, sh.d0s);
                 else if (mode == 2u) walk_span<2u, true>(p, R, x6[h].x, xs, xe, pi0, w0, w1, w2, sh.key, sh.d0s);
+                else if (p.depth_test == DT_NONE) walk_span<3u, true>(p, R, x6[h].x, xs, xe, pi0, w0, w1, w2, sh.key, sh.d0s);
                 else walk_span<0u>(p, R, x6[h].x, xs, xe, pi0, w0, w1, w2, sh.key, sh.d0s);
             }
         }
