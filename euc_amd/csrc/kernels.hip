@@ -787,6 +787,11 @@ EUCHIP_DEV uint64_t init_key(uint32_t mode, float D0) {
     return (uint64_t)o << 32;
 }
 
+// The winning primitive + 1 of a key, 0 where there is none.
+EUCHIP_DEV uint32_t key_prim(uint32_t mode, uint64_t kk) {
+    return mode == 0u ? (uint32_t)(kk >> 32) : (uint32_t)kk >> 1;
+}
+
 EUCHIP_DEV void update_key(uint64_t *key, uint32_t mode, uint32_t test, float z, float D0, uint32_t prim) {
     if (mode == 0u) {
         bool pass;
@@ -862,53 +867,21 @@ EUCHIP_DEV void v_data(const TriRec &R, const float (*V)[VDN<SH>::N], float X, f
     }
 }
 
-// Deferred shading of one pixel's winning fragment (pipeline.rs:539-576).
-// MS: the frame's MSAA level is above 0 (coarse shading); the one-sample and
-// the coarse kernels are compiled apart so the first keep the registers the
-// second needs for its four samples.
-template <uint32_t SH, bool GS, bool MS>
-EUCHIP_DEV uint32_t shade_pixel(const FrameParams &p, const View &v, const TriRec &R, uint32_t px, uint32_t py,
-                                uint32_t by0, uint32_t old) {
+// VertexData of a record's corners, interpolated at (X, Y), through the fragment
+// shader: the deferred shading of a winning fragment (pipeline.rs:539-541), or
+// one coarse sample of it (pipeline.rs:541-570).
+template <uint32_t SH, bool GS>
+EUCHIP_DEV void shade_sample(const FrameParams &p, const View &v, const TriRec &R, float X, float Y, float frag[4]) {
     constexpr uint32_t NV = VDN<SH>::N;
-    float V[3][NV];
+    float V[3][NV], vd[NV];
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         const float *src = p.vary + (size_t)R.sid[i] * vd_count(SH);
 #pragma unroll
         for (uint32_t c = 0; c < vd_count(SH); c++) V[i][c] = src[c];
     }
-    float frag[4], vd[NV];
-    const uint32_t L = p.msaa_level;
-    if constexpr (!MS) {
-        v_data<SH>(R, V, (float)px, (float)py, vd);
-        fragment_shader<SH, GS>(v, p.sampler, vd, frag);
-    } else {
-        // coarse shading on the band-relative 2^L grid with bilinear reconstruction
-        // (pipeline.rs:541-570); tgt_min = (0, by0)
-        const float div = 1.0f / (float)(1u << L);
-        const uint32_t rx = px, ry = py - by0;
-        const float fx = rfract((float)rx * div);
-        const float fy = rfract((float)ry * div);
-        const uint32_t cx = rx >> L, cy = ry >> L;
-        float t[4][4];  // t00, t10, t01, t11
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t ix = cx + (uint32_t)(q & 1), iy = cy + (uint32_t)(q >> 1);
-            v_data<SH>(R, V, (float)(ix << L), (float)(by0 + (iy << L)), vd);
-            fragment_shader<SH, GS>(v, p.sampler, vd, t[q]);
-        }
-        if constexpr (SH == FLAT) {
-            frag[0] = t[0][0];
-        } else {
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const float t0 = t[0][c] * (1.0f - fy) + t[2][c] * fy;
-                const float t1 = t[1][c] * (1.0f - fy) + t[3][c] * fy;
-                frag[c] = t0 * (1.0f - fx) + t1 * fx;
-            }
-        }
-    }
-    return blend_shader<SH>(old, frag, p.bgra);
+    v_data<SH>(R, V, X, Y, vd);
+    fragment_shader<SH, GS>(v, p.sampler, vd, frag);
 }
 
 // Tile geometry: TW x TH pixels at (X0, Y0); TW = 1 << sx, TH = 256 >> sx.
@@ -1124,6 +1097,23 @@ EUCHIP_DEV uint32_t block_inclusive_sum(TileShared &sh, uint32_t tid, uint32_t v
     return incl + carry;
 }
 
+// Rank of this thread among the workgroup's threads with `on`, and their number;
+// every thread must call it.
+EUCHIP_DEV uint32_t block_rank(TileShared &sh, uint32_t tid, bool on, uint32_t &total) {
+    const uint64_t bal = __ballot(on);
+    if ((tid & 63u) == 0u) sh.wave_rows[tid >> 6] = (uint32_t)__popcll(bal);
+    __syncthreads();
+    uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+    total = 0u;
+#pragma unroll
+    for (uint32_t w = 0; w < 4u; w++) {
+        const uint32_t c = sh.wave_rows[w];
+        at += w < (tid >> 6) ? c : 0u;
+        total += c;
+    }
+    return at;
+}
+
 // One batch of up to 256 bin entries: each lane stages its entry's setup in LDS,
 // then the (entry, row) pairs of the batch are spread over all lanes so no
 // lane walks much more than one row.
@@ -1242,18 +1232,16 @@ EUCHIP_DEV void big_tasks(const FrameParams &p, TileShared &sh, uint32_t tid, ui
     }
 }
 
-// Waves per SIMD the raster pass is compiled for (measured per shader): latency
-// hiding pays for a few spilled registers, up to a point.  Without coarse
-// shading every one-request and batched kernel fits these without spills.
-// The big-triangle kernels hold two row tasks per lane and take 6 (their
-// frames have few tiles, so fewer waves per SIMD than that are resident anyway).
-constexpr uint32_t raster_waves(uint32_t sh, bool ms, bool big) {
-    return ms ? ((sh == PHONG_SHADOW || sh == TEX_SHADOW) ? 5u : sh == TEXTURED ? 7u : (sh == DEPTH_ONLY || sh == FLAT) ? 8u : 7u)
-              : big ? 6u : ((sh == PHONG_SHADOW || sh == TEX_SHADOW) ? 7u : 8u);
+// Waves per SIMD the raster pass is compiled for: what its registers allow
+// without spills.  The big-triangle kernels hold two row tasks per lane and take
+// 6 (their frames have few tiles, so fewer waves per SIMD than that are resident
+// anyway).
+constexpr uint32_t raster_waves(uint32_t sh, bool big) {
+    return big ? 6u : (sh == PHONG_SHADOW || sh == TEX_SHADOW) ? 7u : 8u;
 }
 
 template <uint32_t SH, bool BATCH, bool BIG, bool GS, bool MS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(SH, MS, BIG)))) void k_raster(FrameParams) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(SH, BIG)))) void k_raster(FrameParams) {
     __shared__ TileShared sh;
     warm_args();
     const uint32_t tid = threadIdx.x;
@@ -1454,34 +1442,92 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
                 }
             }
         }
-        // The pixels to shade, packed onto the first lanes in tile order: a wave
-        // with none of them skips the shader.
-        if constexpr (SH != DEPTH_ONLY) {
-            const uint64_t bal = __ballot(shade);
-            if ((tid & 63u) == 0u) sh.wave_rows[tid >> 6] = (uint32_t)__popcll(bal);
-            __syncthreads();
-            uint32_t at = 0, total = 0;
-#pragma unroll
-            for (uint32_t w4 = 0; w4 < 4u; w4++) {
-                const uint32_t c = sh.wave_rows[w4];
-                at += w4 < (tid >> 6) ? c : 0u;
-                total += c;
-            }
-            if (shade) sh.owner[at + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = (uint8_t)tid;
+        if constexpr (SH != DEPTH_ONLY && (!MS || SH == FLAT)) {  // (FLAT is the same at every coarse sample)
+            // The pixels to shade, packed onto the first lanes in tile order: a wave
+            // with none of them skips the shader.
+            uint32_t total;
+            const uint32_t at = block_rank(sh, tid, shade, total);
+            if (shade) sh.owner[at] = (uint8_t)tid;
             __syncthreads();
             if (tid < total) {
                 const FrameParams &p = args();
                 const View &v = view_of<BATCH>(p, r);
                 const uint32_t t = sh.owner[tid];
                 const uint32_t tx2 = g.X0 + (t & (g.TW - 1u)), ty2 = g.Y0 + (t >> sx);
-                const uint64_t kk = sh.key[t + (t >> sx)];
-                const uint32_t prim = key_mode(p) == 0u ? (uint32_t)(kk >> 32) - 1u : ((uint32_t)kk >> 1) - 1u;
+                const uint32_t prim = key_prim(key_mode(p), sh.key[t + (t >> sx)]) - 1u;
                 TriRec R;
                 load_rec0(p, tri_base + prim, R);
                 tri_sids(v, p.geometry, prim, R.flags, R.sid);
-                store_stream(&v.pixel[(size_t)ty2 * v.W + tx2],
-                             shade_pixel<SH, GS, MS>(p, v, R, tx2, ty2, sh.band[2 * (t >> sx)],
-                                                     v.clear_color_en ? v.clear_color : 0u));
+                float frag[4];
+                shade_sample<SH, GS>(p, v, R, (float)tx2, (float)ty2, frag);
+                store_stream(&v.pixel[(size_t)ty2 * v.W + tx2], blend_shader<SH>(0u, frag, p.bgra));
+            }
+        } else if constexpr (SH != DEPTH_ONLY) {
+            // Coarse shading (pipeline.rs:541-570): a pixel combines four samples of
+            // its winner at the corners of its cell of the band's 2^L grid.  Pixels
+            // of a cell with the same winner have the same samples; a 2 x 2 block
+            // of even band rows and columns always lies in one cell, so the samples
+            // are taken once per block and winner: its first pixel leads.  Each lane
+            // takes one sample of a leader, 64 leaders a round, into LDS, and the
+            // pixels combine them.  (With four samples per pixel and lane the
+            // 1080p terrain's main pass spent three quarters of its vector
+            // instructions on samples that its neighbours took as well.)
+            const uint32_t mode = key_mode(args());
+            const uint32_t tx = tid & (g.TW - 1u), ty = tid >> sx;
+            const uint32_t by0 = sh.band[2 * ty], pid = shade ? key_prim(mode, sh.key[tid + ty]) : 0u;
+            uint32_t leader = tid;
+            if (shade) {
+                const uint32_t odd = (g.Y0 + ty - by0) & 1u;  // second row of its block
+                const uint32_t x0 = tx & ~1u, row = odd ? ty - 1u : ty;
+                const bool above = odd && ty > 0u;  // its first row is in this tile (and then in this band)
+                if (tx & 1u && key_prim(mode, sh.key[ty * (g.TW + 1u) + x0]) == pid) leader = (ty << sx) + x0;
+                if (above) {
+                    if (key_prim(mode, sh.key[row * (g.TW + 1u) + x0 + 1u]) == pid) leader = (row << sx) + x0 + 1u;
+                    if (key_prim(mode, sh.key[row * (g.TW + 1u) + x0]) == pid) leader = (row << sx) + x0;
+                }
+            }
+            uint32_t total;
+            const uint32_t at = block_rank(sh, tid, shade && leader == tid, total);
+            if (shade && leader == tid) sh.owner[at] = (uint8_t)tid, sh.rows_incl[tid] = at;
+            __syncthreads();
+            const uint32_t mine = shade ? sh.rows_incl[leader] : ~0u;  // the leader's rank
+            float4 *const sample = reinterpret_cast<float4 *>(sh.tri);
+            static_assert(sizeof(sh.tri) >= 256u * sizeof(float4), "a round's samples fit the staging space");
+            for (uint32_t b = 0; b < total; b += 64u) {
+                const FrameParams &p = args();
+                const View &v = view_of<BATCH>(p, r);
+                const uint32_t L = p.msaa_level;
+                if (b + (tid >> 2) < total) {
+                    const uint32_t t = sh.owner[b + (tid >> 2)], q = tid & 3u;
+                    const uint32_t prim = key_prim(mode, sh.key[t + (t >> sx)]) - 1u;
+                    const uint32_t b0 = sh.band[2 * (t >> sx)];
+                    const uint32_t cx = (g.X0 + (t & (g.TW - 1u))) >> L, cy = (g.Y0 + (t >> sx) - b0) >> L;
+                    TriRec R;
+                    load_rec0(p, tri_base + prim, R);
+                    tri_sids(v, p.geometry, prim, R.flags, R.sid);
+                    float frag[4];
+                    shade_sample<SH, GS>(p, v, R, (float)((cx + (q & 1u)) << L), (float)(b0 + ((cy + (q >> 1)) << L)), frag);
+                    sample[tid] = make_float4(frag[0], frag[1], frag[2], frag[3]);
+                }
+                __syncthreads();
+                if (mine - b < 64u) {
+                    // bilinear reconstruction (pipeline.rs:556-570)
+                    const float div = 1.0f / (float)(1u << L);
+                    const float fx = rfract((float)(g.X0 + tx) * div), fy = rfract((float)(g.Y0 + ty - by0) * div);
+                    const float4 *s4 = sample + 4u * (mine - b);  // t00, t10, t01, t11
+                    const float4 t00 = s4[0], t10 = s4[1], t01 = s4[2], t11 = s4[3];
+                    const float c00[4] = {t00.x, t00.y, t00.z, t00.w}, c10[4] = {t10.x, t10.y, t10.z, t10.w};
+                    const float c01[4] = {t01.x, t01.y, t01.z, t01.w}, c11[4] = {t11.x, t11.y, t11.z, t11.w};
+                    float frag[4];
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const float t0 = c00[c] * (1.0f - fy) + c01[c] * fy;
+                        const float t1 = c10[c] * (1.0f - fy) + c11[c] * fy;
+                        frag[c] = t0 * (1.0f - fx) + t1 * fx;
+                    }
+                    store_stream(&v.pixel[(size_t)(g.Y0 + ty) * v.W + g.X0 + tx], blend_shader<SH>(0u, frag, p.bgra));
+                }
+                __syncthreads();  // the next round's samples reuse the space
             }
         }
         __syncthreads();
