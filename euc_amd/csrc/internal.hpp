@@ -216,6 +216,7 @@ struct View {
     Divisor inst_tris;     // triangles per instance (INST_TRIANGLES)
     Divisor inst_verts;    // vertices per instance
     Divisor row_tiles;     // ntx
+    Divisor row_pixels;    // W (lines)
     // textures (device)
     gptr<const uint32_t> tex;
     uint32_t tex_w, tex_h;
@@ -238,9 +239,10 @@ struct FrameParams {
     uint32_t sampler;      // texture sampler kind (resolved: never EUCHIP_SAMPLER_DEFAULT)
     uint32_t geometry;     // Geometry: primitive t of the stream is stage output t % k of input triangle t / k
     // lines (one-request frames): LINE_LIST or LINE_TRIANGLE_LIST, n_lines lines;
-    // a 64-byte record per line and a 64-bit winner key per target pixel
+    // per line what its pixels' shading reads, per target pixel a 64-bit winner
+    // key, zero between frames
     uint32_t primitives, n_lines;
-    gptr<uint32_t> lrec;
+    gptr<uint4> lrec;
     gptr<uint64_t> lkey;
     // per-launch scratch (device)
     gptr<uint4> rec0;           // kRec0Quads per triangle of the launch
@@ -331,14 +333,14 @@ hipError_t launch_raster(const FrameParams &p, hipStream_t s, bool batched);
 // Row checkpoints of the big triangles (one-request big-triangle frames with a
 // checkpoint pool), between setup and raster.
 hipError_t launch_fill_u32(uint32_t *dst, uint32_t value, size_t n, hipStream_t s);
-// The lines path of one request (p.v0): vertex stage + line setup, winner keys
-// initialised, lines walked, then every pixel resolved (colour, depth, clears).
+// The lines path of one request (p.v0): vertex stage beside line setup and walk,
+// then every pixel resolved (colour, depth, clears).
 hipError_t launch_lines(const FrameParams &p, hipStream_t s);
 
 // PrimitiveKind (EUCHIP_PRIMS_*).
 enum Prims : uint32_t { PRIMS_TRIANGLES = 0, PRIMS_LINE_LIST = 1, PRIMS_LINE_TRIANGLES = 2 };
 // Line endpoints further than this from the origin (pixels) are not drawn.
 constexpr int32_t kLineCoordLimit = 1 << 29;
-constexpr uint32_t kLineRecWords = 16;
+constexpr uint32_t kLineRecQuads = 2;
 
 }  // namespace euchip

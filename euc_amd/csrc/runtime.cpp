@@ -73,8 +73,9 @@ struct euchip_ctx {
     DevArray<uint2> cktab;     // per tile: its list of (triangle, row mask; key-order bound)
     DevArray<uint2> ck_count;  // the lists' lengths and occluder bounds, two halves like tile_count
     uint32_t ck_dirty[2] = {0, 0};  // counts a checkpoint frame left in each half, zeroed by the next frame
-    DevArray<uint32_t> lrec;    // line records
-    DevArray<uint64_t> lkey;    // per-pixel winner keys of a lines frame
+    DevArray<uint4> lrec;       // line records
+    DevArray<uint64_t> lkey;    // per-pixel winner keys of a lines frame, zero between frames
+    bool lkey_clean = false;    // all of lkey is zero once the enqueued frames are done
     std::vector<Deferred> deferred;
     uint32_t counts_used[2] = {0, 0};  // tiles of the last frame that counted into each half of tile_count
     uint32_t tile_cap = 128;    // bin slots per tile; raised when a frame needed more (within the bin budget)
@@ -514,14 +515,26 @@ euchip_status render_lines(euchip_ctx *ctx, const euchip_pipeline_desc *d, const
     const size_t npx = (size_t)P.v.W * P.v.H;
     if ((s = ensure(ctx, ctx->vary, std::max<size_t>(P.n_sv * vd_count(d->shader), 1), "vertex data", ctx->stream)))
         return s;
-    if ((s = ensure(ctx, ctx->lrec, std::max<size_t>((size_t)p.n_lines * kLineRecWords, 1), "line records",
+    if ((s = ensure(ctx, ctx->lrec, std::max<size_t>((size_t)p.n_lines * kLineRecQuads, 1), "line records",
                     ctx->stream)))
         return s;
-    if ((s = ensure(ctx, ctx->lkey, npx, "line keys", ctx->stream))) return s;
+    const uint64_t *keys_had = ctx->lkey.ptr;
+    if ((s = ensure(ctx, ctx->lkey, npx, "line keys", ctx->stream))) {
+        ctx->lkey_clean = false;  // (the old storage is gone)
+        return s;
+    }
+    // new storage starts at zero, as every frame leaves it; after a frame that
+    // was not enqueued whole it starts over
+    if (ctx->lkey.ptr != keys_had) ctx->lkey_clean = false;
+    if (!ctx->lkey_clean)
+        HIP_TRY(ctx, launch_fill_u32((uint32_t *)ctx->lkey.ptr, 0u, 2 * ctx->lkey.cap, ctx->stream));
+    ctx->lkey_clean = false;
+    p.v0.row_pixels = make_divisor(P.v.W);
     p.vary = ctx->vary.ptr;
     p.lrec = ctx->lrec.ptr;
     p.lkey = ctx->lkey.ptr;
     if ((s = timed(ctx, "lines", [&] { return launch_lines(p, ctx->stream); }))) return s;
+    ctx->lkey_clean = true;
     if (sync) {
         HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->profiling) resolve_pending(ctx);

@@ -1,0 +1,58 @@
+"""The lines' walk and the keys between frames, against the oracle, bit-exact:
+lines of one pixel, of about the length at which the whole wave takes a line, far
+longer, and with ends thousands of pixels outside (64-bit steps), line counts
+around a workgroup's 16; and frames of other depth modes, sizes and loaded
+targets after one another on one context, which find the keys of the last frame
+zeroed."""
+import numpy as np
+import pytest
+
+from euc_amd import scenes as S
+from euc_amd.pipeline import BandPolicy, DepthMode, PipelineDesc, Primitives, Shader, Xform
+from euc_amd.renderer import Context
+from tests.parity import assert_bit_exact, run_pair
+
+pytestmark = pytest.mark.gpu
+
+
+def lines(seed, n, length, w, extent=1.0):
+    """n lines of about `length` pixels at a target of width w."""
+    rng = np.random.default_rng(seed)
+    pos = np.ones((n, 2, 4), np.float32)
+    pos[:, 0, :2] = rng.uniform(-extent, extent, (n, 2))
+    pos[:, 1, :2] = pos[:, 0, :2] + rng.normal(0.0, 2.0 * length / w, (n, 2))
+    pos[:, :, 2] = rng.uniform(0.0, 1.0, (n, 2))
+    rgba8 = rng.integers(0, 2 ** 32, 2 * n, dtype=np.uint64).astype(np.uint32)
+    return S.Mesh(pos=pos.reshape(-1, 4), count=2 * n, rgba8=rgba8)
+
+
+def desc(dm, band=BandPolicy.SEQ):
+    return PipelineDesc.make(Shader.FLAT, Xform.CLIP, depth_mode=dm, band_policy=band, primitives=Primitives.LINE_LIST)
+
+
+@pytest.mark.parametrize("n,length,extent", [(1, 20, 0.5), (15, 1, 1.0), (17, 255, 0.8), (64, 260, 1.0), (300, 900, 1.5),
+                                             (40, 60000, 30.0), (4000, 12, 1.0)])
+def test_line_lengths(gpu_ctx, n, length, extent):
+    w, h = 1500, 700
+    mesh = lines(n + length, n, length, w, extent)
+    r = run_pair(gpu_ctx, desc(DepthMode.LESS_WRITE), S.uniforms(), mesh, w, h)
+    assert_bit_exact(r, f"{n} lines of {length}")
+
+
+def test_keys_between_frames():
+    ctx = Context(0)
+    try:
+        rng = np.random.default_rng(3)
+        for k, (dm, w, h, load) in enumerate([
+                (DepthMode.LESS_WRITE, 300, 200, False), (DepthMode.GREATER_WRITE, 300, 200, True),
+                (DepthMode.NONE, 640, 480, False), (DepthMode.LESS_PASS, 200, 333, True),
+                (DepthMode.LESS_WRITE, 640, 480, True), (DepthMode.NONE, 64, 48, True),
+                (DepthMode.GREATER_PASS, 900, 600, True), (DepthMode.LESS_WRITE, 300, 200, False)]):
+            mesh = lines(50 + k, 500, 60, w)
+            z = rng.uniform(0.2, 0.8, (h, w)).astype(np.float32) if load else 1.0
+            c = rng.integers(0, 2 ** 32, (h, w), dtype=np.uint64).astype(np.uint32) if load else 7
+            r = run_pair(ctx, desc(dm), S.uniforms(), mesh, w, h, color_init=c, depth_init=z)
+            assert r["frags"] > 50
+            assert_bit_exact(r, f"frame {k} {dm}")
+    finally:
+        ctx.close()
