@@ -1939,6 +1939,10 @@ struct LineWalk {
 
 // Steps k = klo + first, klo + first + stride, ... of line l: each pixel's key is
 // raised by its fragment (key 0: no fragment; the greatest key wins).
+// LOADS: a depth test reads the target's depth before the pass (not the clear's).
+// Kernels of their own: a loop that may load waits in every step for the step
+// before's atomic.
+template <bool LOADS>
 EUCHIP_DEV void walk_line(const FrameParams &p, const View &v, uint32_t l, const LineWalk &W, uint32_t first, uint32_t stride) {
     const uint32_t mode = key_mode(p);
     for (int32_t k = W.klo + (int32_t)first; k <= W.khi; k += (int32_t)stride) {
@@ -1955,8 +1959,7 @@ EUCHIP_DEV void walk_line(const FrameParams &p, const View &v, uint32_t l, const
         if (!passes_z_clip(p, z)) continue;
         const size_t pi = (size_t)y * v.W + x;
         if (p.depth_test != DT_NONE) {
-            float D0 = v.clear_depth;
-            if (!v.clear_depth_en) D0 = v.depth[pi];
+            const float D0 = LOADS ? v.depth[pi] : v.clear_depth;
             if (!(p.depth_test == DT_LESS ? z < D0 : p.depth_test == DT_EQUAL ? z == D0 : z > D0)) continue;
         }
         // the keys of init_key, those of the write modes complemented
@@ -1980,7 +1983,7 @@ EUCHIP_DEV void walk_line(const FrameParams &p, const View &v, uint32_t l, const
 constexpr uint32_t kLinesPerBlock = 16;
 constexpr int32_t kLongLine = 256;
 
-template <uint32_t SH>
+template <uint32_t SH, bool LOADS>
 __global__ __launch_bounds__(256) void k_line_draw(FrameParams) {
     warm_args();
     const FrameParams &p = args();
@@ -2056,7 +2059,7 @@ __global__ __launch_bounds__(256) void k_line_draw(FrameParams) {
         }
     }
     const bool wide = W.khi - W.klo >= kLongLine;
-    if (!wide) walk_line(p, v, l, W, tid & 15u, 16u);
+    if (!wide) walk_line<LOADS>(p, v, l, W, tid & 15u, 16u);
     for (uint64_t m = __ballot(wide) & 0x0001000100010001ull; m; m &= m - 1u) {
         const int g = __ffsll((unsigned long long)m) - 1;  // the line's first lane
         auto bi = [&](int32_t q) { return __builtin_amdgcn_readlane(q, g); };
@@ -2067,7 +2070,7 @@ __global__ __launch_bounds__(256) void k_line_draw(FrameParams) {
         B.n0 = bi(W.n0), B.n1 = bi(W.n1), B.klo = bi(W.klo), B.khi = bi(W.khi);
         B.xmajor = bu(W.xmajor) != 0u, B.use_x = bu(W.use_x) != 0u;
         B.vs0 = bf(W.vs0), B.norm = bf(W.norm), B.ez0 = bf(W.ez0), B.ez1 = bf(W.ez1);
-        walk_line(p, v, bu(l), B, lane_id(), 64u);
+        walk_line<LOADS>(p, v, bu(l), B, lane_id(), 64u);
     }
 }
 
@@ -2169,7 +2172,10 @@ static void launch_lines_t(const FrameParams &p, hipStream_t s) {
     FrameParams q = p;
     q.tri_blocks = blocks_of(p.n_lines, kLinesPerBlock);
     const uint32_t blocks = q.tri_blocks + (vd_count(SH) > 0 ? blocks_of(nsv, 256) : 0u);
-    hipLaunchKernelGGL((k_line_draw<SH>), dim3(blocks), dim3(256), 0, s, q);
+    if (p.depth_test != DT_NONE && !p.v0.clear_depth_en)
+        hipLaunchKernelGGL((k_line_draw<SH, true>), dim3(blocks), dim3(256), 0, s, q);
+    else
+        hipLaunchKernelGGL((k_line_draw<SH, false>), dim3(blocks), dim3(256), 0, s, q);
     hipLaunchKernelGGL((k_line_resolve<SH>), dim3(blocks_of(npx, 256)), dim3(256), 0, s, q);
 }
 
