@@ -1319,6 +1319,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         if (!for_heavy && w >= nbusy) tile = ~0u;
     }
 
+    // This workgroup's tile of the XCD's range where it is empty (launches of more
+    // tiles than workgroups: its tiles): the clears, stores only.
+    for (uint32_t ctile = t0 + w; clears;) {
+        if (count == 0u) {
+            const FrameParams &p = args();
+            const uint32_t sx = p.tile_sx;
+            uint32_t r = 0;
+            if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(uniform_load(p.tile_req + ctile));
+            const View &v = view_of<BATCH>(p, r);
+            const uint32_t lt = ctile - v.tile_base;
+            const uint32_t ty = divide(lt, v.row_tiles), tx = lt - ty * v.ntx;
+            const uint32_t px = (tx << sx) + (tid & ((1u << sx) - 1u)), py = (ty << (8u - sx)) + (tid >> sx);
+            if (px < v.W && py < v.H) {
+                const size_t pidx = (size_t)py * v.W + px;
+                if (v.pixel && v.clear_color_en) store_stream(&v.pixel[pidx], v.clear_color);
+                if (v.depth && v.clear_depth_en) store_stream(&v.depth[pidx], v.clear_depth);
+            }
+        }
+        if (t1 - ctile <= per_xcd) break;
+        ctile += per_xcd;
+        count = uniform_load(&args().tile_count[ctile].count);
+    }
+
     // One tile with `cnt` bin entries and overflow list `head`: winner keys in
     // LDS, then the resolve.  Ends with a barrier (LDS is reused by a next tile).
     // Loads the bin state `ntb` of the workgroup's next tile on the way.
@@ -1538,19 +1561,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
     // at the start of a tile, its bin state before the resolve.
     const bool heavy = blockIdx.x < args().heavy_groups;
     uint32_t k = heavy ? blockIdx.x : w;
+    const uint32_t stride = heavy ? args().heavy_groups : per_xcd, bound = heavy ? nh : nbusy;
     TileBin tb = tile != ~0u ? uniform_load(&args().tile_count[tile]) : TileBin{0u, 0u};
     while (tile != ~0u) {
         uint32_t ntile = ~0u;
-        {
+        k += stride;
+        if (k < bound) {
             const FrameParams &p = args();
-            k += heavy ? p.heavy_groups : per_xcd;
-            if (k < (heavy ? nh : nbusy)) {
-                uint32_t lbase, lcap;
-                busy_list_span(p, xcd, lbase, lcap);
-                if (heavy) ntile = uniform_load(p.heavy + k);
-                else if (BIG && nbig) ntile = t0 + k;
-                else ntile = uniform_load(p.busy + lbase + k);
-            }
+            uint32_t lbase, lcap, b0, b1;
+            busy_list_span(p, xcd, lbase, lcap);
+            xcd_range(p.ntiles, xcd, b0, b1);
+            if (heavy) ntile = uniform_load(p.heavy + k);
+            else if (BIG && nbig) ntile = b0 + k;
+            else ntile = uniform_load(p.busy + lbase + k);
         }
         TileBin ntb{0u, 0u};
         if (heavy || !args().heavy_cap || tb.count < kHeavyTile)
@@ -1558,29 +1581,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         else if (ntile != ~0u)  // a heavy tile of the busy list: another workgroup's
             ntb = uniform_load(&args().tile_count[ntile]);
         tile = ntile, tb = ntb;
-    }
-    // This workgroup's tile of the XCD's range where it is empty (launches of more
-    // tiles than workgroups: its tiles): the clears, stores only.
-    if (!clears) return;
-    for (uint32_t tile = t0 + w;;) {
-        if (count == 0u) {
-            const FrameParams &p = args();
-            const uint32_t sx = p.tile_sx;
-            uint32_t r = 0;
-            if constexpr (BATCH) r = __builtin_amdgcn_readfirstlane(uniform_load(p.tile_req + tile));
-            const View &v = view_of<BATCH>(p, r);
-            const uint32_t lt = tile - v.tile_base;
-            const uint32_t ty = divide(lt, v.row_tiles), tx = lt - ty * v.ntx;
-            const uint32_t px = (tx << sx) + (tid & ((1u << sx) - 1u)), py = (ty << (8u - sx)) + (tid >> sx);
-            if (px < v.W && py < v.H) {
-                const size_t pidx = (size_t)py * v.W + px;
-                if (v.pixel && v.clear_color_en) store_stream(&v.pixel[pidx], v.clear_color);
-                if (v.depth && v.clear_depth_en) store_stream(&v.depth[pidx], v.clear_depth);
-            }
-        }
-        if (t1 - tile <= per_xcd) break;
-        tile += per_xcd;
-        count = uniform_load(&args().tile_count[tile].count);
     }
 }
 

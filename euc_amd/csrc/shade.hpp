@@ -34,12 +34,9 @@ EUCHIP_DEV uint32_t sat_clamp(float f, uint32_t lo, uint32_t hi) {
     return v < lo ? lo : v;
 }
 
-// `f as u8`: saturating truncation, NaN -> 0.
-EUCHIP_DEV uint32_t sat_u8(float f) {
-    if (!(f > 0.0f)) return 0;
-    if (f >= 255.0f) return 255;
-    return (uint32_t)f;
-}
+// `f as u8`: saturating truncation, NaN -> 0 (rmax takes the other operand, and
+// a value in [0, 255] only truncates).
+EUCHIP_DEV uint32_t sat_u8(float f) { return (uint32_t)rmin(rmax(f, 0.0f), 255.0f); }
 
 template <class M>  // a matrix in any memory
 EUCHIP_DEV void mat4_vec4(const M *m, const float v[4], float r[4]) {
@@ -319,7 +316,7 @@ EUCHIP_DEV uint32_t blend_shader(uint32_t old, const float f[4], uint32_t bgra) 
         for (int c = 0; c < 4; c++) b[c] = sat_u8(f[c]);
     } else {
 #pragma unroll
-        for (int c = 0; c < 4; c++) b[c] = sat_u8(rmin(rmax(f[c], 0.0f), 1.0f) * 255.0f);
+        for (int c = 0; c < 4; c++) b[c] = (uint32_t)(rmin(rmax(f[c], 0.0f), 1.0f) * 255.0f);  // in [0, 255]: no saturation
     }
     if (bgra) return b[2] | (b[1] << 8) | (b[0] << 16) | (b[3] << 24);
     return b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
