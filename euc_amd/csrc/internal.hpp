@@ -123,6 +123,20 @@ enum BusyMap : uint32_t { BUSY_RANGES = 0, BUSY_BLOCKS = 1 };
 constexpr uint32_t kBigTiles = 64;
 constexpr uint32_t kBigCap = 4096;
 
+// One-request frames of few triangles on targets that are not too wide take one
+// launch (k_tiny) of at most kTinyGroups workgroups, no scratch memory and no
+// frame number: at most kTinyTris triangles, kTinyWidth columns, and triangles x
+// columns^2 (what walking every row from its start costs per row) at most
+// kTinyWork.  Against a checkpoint frame, us per pass: a cube of 12 triangles 36.0 /
+// 26.3 at 800 columns, 60.8 / 38.8 at 1600 (135 / 95 at 3200, but not where
+// triangles fill the target); triangles that each fill it, the worst case: 16 of
+// them 26 / 17 at 640 columns and 50 / 48 at 1280, 64 of them 31 / 32 at 640 and 55
+// / 113 at 1280, 2 of them 49 / 39 at 1280 and 79 / 91 at 1920.
+constexpr uint32_t kTinyTris = 64;
+constexpr uint32_t kTinyWidth = 1600;
+constexpr uint64_t kTinyWork = (uint64_t)12 * 1600 * 1600;
+constexpr uint32_t kTinyGroups = 1536;  // what the compute units hold at once (6 each)
+
 // Row checkpoints of big triangles.  The exact walk of a row (w += dx from the
 // row start x0, triangles.rs:257-301) reaches a tile only after every pixel
 // left of it; the span blocks of the setup launch walk each row of each big
@@ -330,6 +344,8 @@ hipError_t noalloc_scratch(int device, void **out);
 // workgroups as p.blk maps them); one-request launches read p.v0.
 hipError_t launch_setup(const FrameParams &p, hipStream_t s, bool batched, uint32_t blocks);
 hipError_t launch_raster(const FrameParams &p, hipStream_t s, bool batched);
+// The whole frame of a small mesh (p.v0): setup and raster in one launch.
+hipError_t launch_tiny(const FrameParams &p, hipStream_t s);
 // Row checkpoints of the big triangles (one-request big-triangle frames with a
 // checkpoint pool), between setup and raster.
 hipError_t launch_fill_u32(uint32_t *dst, uint32_t value, size_t n, hipStream_t s);

@@ -27,6 +27,7 @@
 //             row exactly as triangles.rs:219-303 does (big triangles from
 //             their checkpoints).  The winner is then shaded once and colour
 //             and depth are written once per pixel.
+//   k_tiny    setup and raster of a small mesh in one launch.
 //   k_line_*  the lines rasteriser (lines.rs:15-121) for one request.
 #include "internal.hpp"
 #include "shade.hpp"
@@ -871,15 +872,9 @@ EUCHIP_DEV void v_data(const TriRec &R, const float (*V)[VDN<SH>::N], float X, f
 // shader: the deferred shading of a winning fragment (pipeline.rs:539-541), or
 // one coarse sample of it (pipeline.rs:541-570).
 template <uint32_t SH, bool GS>
-EUCHIP_DEV void shade_sample(const FrameParams &p, const View &v, const TriRec &R, float X, float Y, float frag[4]) {
-    constexpr uint32_t NV = VDN<SH>::N;
-    float V[3][NV], vd[NV];
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const float *src = p.vary + (size_t)R.sid[i] * vd_count(SH);
-#pragma unroll
-        for (uint32_t c = 0; c < vd_count(SH); c++) V[i][c] = src[c];
-    }
+EUCHIP_DEV void shade_sample(const FrameParams &p, const View &v, const TriRec &R, const float (*V)[VDN<SH>::N], float X,
+                             float Y, float frag[4]) {
+    float vd[VDN<SH>::N];
     v_data<SH>(R, V, X, Y, vd);
     fragment_shader<SH, GS>(v, p.sampler, vd, frag);
 }
@@ -1062,6 +1057,14 @@ struct TileShared {
     uint32_t band[2 * kMaxTileH];   // [by0, by1) of the render_par band of each row
 };
 
+EUCHIP_DEV void put_tri(TriLds &T, const TriRec &R, uint32_t prim) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) T.o[i] = R.o[i], T.dx[i] = R.dx[i], T.dy[i] = R.dy[i], T.hz[i] = R.hz[i];
+#pragma unroll
+    for (int i = 0; i < 6; i++) T.vby[i] = R.vby[i];
+    T.xmin = R.xmin, T.xmax = R.xmax, T.ymin = R.ymin, T.ymax = R.ymax, T.flags = R.flags, T.prim = prim;
+}
+
 // Rows of bin entry `prim` inside the tile, its setup kept in sh.tri[slot].
 EUCHIP_DEV uint32_t stage_entry(const FrameParams &p, uint32_t tri_base, TileShared &sh, uint32_t slot, uint32_t prim,
                                 const TileGeom &g) {
@@ -1078,12 +1081,7 @@ EUCHIP_DEV uint32_t stage_entry(const FrameParams &p, uint32_t tri_base, TileSha
 #pragma unroll
         for (int i = 0; i < 6; i++) R.vby[i] = 0.0f;  // boxed rows never read verts_by_y
     }
-    TriLds &T = sh.tri[slot];
-#pragma unroll
-    for (int i = 0; i < 3; i++) T.o[i] = R.o[i], T.dx[i] = R.dx[i], T.dy[i] = R.dy[i], T.hz[i] = R.hz[i];
-#pragma unroll
-    for (int i = 0; i < 6; i++) T.vby[i] = R.vby[i];
-    T.xmin = R.xmin, T.xmax = R.xmax, T.ymin = R.ymin, T.ymax = R.ymax, T.flags = R.flags, T.prim = prim;
+    put_tri(sh.tri[slot], R, prim);
     return ry1 - ry0;
 }
 
@@ -1114,15 +1112,13 @@ EUCHIP_DEV uint32_t block_rank(TileShared &sh, uint32_t tid, bool on, uint32_t &
     return at;
 }
 
-// One batch of up to 256 bin entries: each lane stages its entry's setup in LDS,
-// then the (entry, row) pairs of the batch are spread over all lanes so no
-// lane walks much more than one row.
+// The rows of up to kBatch triangles staged in LDS, `rows` of this lane's inside
+// the tile: the (triangle, row) pairs are spread over all lanes so no lane walks
+// much more than one row.  Ends with a barrier.
 template <bool OWNER, bool LONG_ROWS>
-EUCHIP_DEV void raster_batch(uint32_t tri_base, TileShared &sh, uint32_t tid, bool valid, uint32_t prim,
-                             const TileGeom &g) {
+EUCHIP_DEV void walk_rows(TileShared &sh, uint32_t tid, uint32_t rows, const TileGeom &g) {
     const FrameParams &p = args();
     const uint32_t mode = key_mode(p);
-    const uint32_t rows = valid ? stage_entry(p, tri_base, sh, tid, prim, g) : 0u;
     const uint32_t incl = block_inclusive_sum(sh, tid, rows);
     const uint32_t excl = incl - rows;
     sh.rows_incl[tid] = incl;
@@ -1158,6 +1154,15 @@ EUCHIP_DEV void raster_batch(uint32_t tri_base, TileShared &sh, uint32_t tid, bo
         raster_row<LONG_ROWS ? 8u : 4u>(p, R, T.prim, ry0 + (k - base), g, mode, sh.key, sh.d0s, sh.band);
     }
     __syncthreads();  // the next batch reuses sh.tri and sh.rows_incl
+}
+
+// One batch of up to 256 bin entries: each lane stages its entry's setup in LDS,
+// then the batch's rows are walked.
+template <bool OWNER, bool LONG_ROWS>
+EUCHIP_DEV void raster_batch(uint32_t tri_base, TileShared &sh, uint32_t tid, bool valid, uint32_t prim,
+                             const TileGeom &g) {
+    const uint32_t rows = valid ? stage_entry(args(), tri_base, sh, tid, prim, g) : 0u;
+    walk_rows<OWNER, LONG_ROWS>(sh, tid, rows, g);
 }
 
 // The big triangles of `tile` from their row checkpoints: the tile's list of
@@ -1229,6 +1234,123 @@ EUCHIP_DEV void big_tasks(const FrameParams &p, TileShared &sh, uint32_t tid, ui
             }
         }
         __syncthreads();  // the next round reuses the table and the wave totals
+    }
+}
+
+// A tile's keys resolved: depth and clears stored, the winners' pixels shaded.
+// view() is the tile's request, read anew for each phase; sample(v, prim, X, Y,
+// frag) is the fragment of primitive prim at (X, Y).
+template <uint32_t SH, bool MS, class ViewF, class SampleF>
+EUCHIP_DEV void resolve_tile(TileShared &sh, uint32_t tid, const TileGeom &g, ViewF view, SampleF sample) {
+    const uint32_t sx = g.sx;
+    bool shade = false;  // this lane's pixel has a winner to shade
+    {
+        const FrameParams &p = args();
+        const View &v = view();
+        const uint32_t mode = key_mode(p);
+        const uint32_t px = g.X0 + (tid & (g.TW - 1u)), py = g.Y0 + (tid >> sx);
+        if (px < v.W && py < v.H) {
+            const size_t pidx = (size_t)py * v.W + px;
+            const uint64_t kk = sh.key[tid + (tid >> sx)];
+            bool has;  // a winner (its primitive is read again by the shading lanes)
+            float z;
+            if (mode == 0u) {
+                has = kk != 0ull;
+                z = __uint_as_float((uint32_t)kk);
+            } else {
+                has = ((uint32_t)kk) != 0u;
+                const uint32_t o = (uint32_t)(kk >> 32);
+                z = zunord(mode == 1u ? o : ~o, (uint32_t)kk & 1u);
+            }
+            shade = v.pixel && p.pixel_write && has && SH != DEPTH_ONLY;
+            if (v.pixel && !shade && v.clear_color_en) store_stream(&v.pixel[pidx], v.clear_color);
+            if (v.depth) {
+                if (has && p.depth_write) store_stream(&v.depth[pidx], z);
+                else if (v.clear_depth_en) store_stream(&v.depth[pidx], v.clear_depth);
+            }
+        }
+    }
+    if constexpr (SH != DEPTH_ONLY && (!MS || SH == FLAT)) {  // (FLAT is the same at every coarse sample)
+        // The pixels to shade, packed onto the first lanes in tile order: a wave
+        // with none of them skips the shader.
+        uint32_t total;
+        const uint32_t at = block_rank(sh, tid, shade, total);
+        if (shade) sh.owner[at] = (uint8_t)tid;
+        __syncthreads();
+        if (tid < total) {
+            const FrameParams &p = args();
+            const View &v = view();
+            const uint32_t t = sh.owner[tid];
+            const uint32_t tx2 = g.X0 + (t & (g.TW - 1u)), ty2 = g.Y0 + (t >> sx);
+            const uint32_t prim = key_prim(key_mode(p), sh.key[t + (t >> sx)]) - 1u;
+            float frag[4];
+            sample(v, prim, (float)tx2, (float)ty2, frag);
+            store_stream(&v.pixel[(size_t)ty2 * v.W + tx2], blend_shader<SH>(0u, frag, p.bgra));
+        }
+    } else if constexpr (SH != DEPTH_ONLY) {
+        // Coarse shading (pipeline.rs:541-570): a pixel combines four samples of
+        // its winner at the corners of its cell of the band's 2^L grid.  Pixels
+        // of a cell with the same winner have the same samples; a 2 x 2 block
+        // of even band rows and columns always lies in one cell, so the samples
+        // are taken once per block and winner: its first pixel leads.  Each lane
+        // takes one sample of a leader, 64 leaders a round, into LDS, and the
+        // pixels combine them.  (With four samples per pixel and lane the
+        // 1080p terrain's main pass spent three quarters of its vector
+        // instructions on samples that its neighbours took as well.)
+        const uint32_t mode = key_mode(args());
+        const uint32_t tx = tid & (g.TW - 1u), ty = tid >> sx;
+        const uint32_t by0 = sh.band[2 * ty], pid = shade ? key_prim(mode, sh.key[tid + ty]) : 0u;
+        uint32_t leader = tid;
+        if (shade) {
+            const uint32_t odd = (g.Y0 + ty - by0) & 1u;  // second row of its block
+            const uint32_t x0 = tx & ~1u, row = odd ? ty - 1u : ty;
+            const bool above = odd && ty > 0u;  // its first row is in this tile (and then in this band)
+            if (tx & 1u && key_prim(mode, sh.key[ty * (g.TW + 1u) + x0]) == pid) leader = (ty << sx) + x0;
+            if (above) {
+                if (key_prim(mode, sh.key[row * (g.TW + 1u) + x0 + 1u]) == pid) leader = (row << sx) + x0 + 1u;
+                if (key_prim(mode, sh.key[row * (g.TW + 1u) + x0]) == pid) leader = (row << sx) + x0;
+            }
+        }
+        uint32_t total;
+        const uint32_t at = block_rank(sh, tid, shade && leader == tid, total);
+        if (shade && leader == tid) sh.owner[at] = (uint8_t)tid, sh.rows_incl[tid] = at;
+        __syncthreads();
+        const uint32_t mine = shade ? sh.rows_incl[leader] : ~0u;  // the leader's rank
+        float4 *const samples = reinterpret_cast<float4 *>(&sh.tri[kTinyTris]);
+        static_assert(sizeof(TriLds) * (kBatch - kTinyTris) >= 256u * sizeof(float4), "a round's samples fit the staging space");
+        for (uint32_t b = 0; b < total; b += 64u) {
+            const FrameParams &p = args();
+            const View &v = view();
+            const uint32_t L = p.msaa_level;
+            if (b + (tid >> 2) < total) {
+                const uint32_t t = sh.owner[b + (tid >> 2)], q = tid & 3u;
+                const uint32_t prim = key_prim(mode, sh.key[t + (t >> sx)]) - 1u;
+                const uint32_t b0 = sh.band[2 * (t >> sx)];
+                const uint32_t cx = (g.X0 + (t & (g.TW - 1u))) >> L, cy = (g.Y0 + (t >> sx) - b0) >> L;
+                float frag[4];
+                sample(v, prim, (float)((cx + (q & 1u)) << L), (float)(b0 + ((cy + (q >> 1)) << L)), frag);
+                samples[tid] = make_float4(frag[0], frag[1], frag[2], frag[3]);
+            }
+            __syncthreads();
+            if (mine - b < 64u) {
+                // bilinear reconstruction (pipeline.rs:556-570)
+                const float div = 1.0f / (float)(1u << L);
+                const float fx = rfract((float)(g.X0 + tx) * div), fy = rfract((float)(g.Y0 + ty - by0) * div);
+                const float4 *s4 = samples + 4u * (mine - b);  // t00, t10, t01, t11
+                const float4 t00 = s4[0], t10 = s4[1], t01 = s4[2], t11 = s4[3];
+                const float c00[4] = {t00.x, t00.y, t00.z, t00.w}, c10[4] = {t10.x, t10.y, t10.z, t10.w};
+                const float c01[4] = {t01.x, t01.y, t01.z, t01.w}, c11[4] = {t11.x, t11.y, t11.z, t11.w};
+                float frag[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const float t0 = c00[c] * (1.0f - fy) + c01[c] * fy;
+                    const float t1 = c10[c] * (1.0f - fy) + c11[c] * fy;
+                    frag[c] = t0 * (1.0f - fx) + t1 * fx;
+                }
+                store_stream(&v.pixel[(size_t)(g.Y0 + ty) * v.W + g.X0 + tx], blend_shader<SH>(0u, frag, p.bgra));
+            }
+            __syncthreads();  // the next round's samples reuse the space
+        }
     }
 }
 
@@ -1437,122 +1559,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             nck = __builtin_amdgcn_readfirstlane(nck);
             if (nck) big_tasks(args(), sh, tid, tile, nck, __builtin_amdgcn_readfirstlane(occl), g, e_first);
         }
-        bool shade = false;  // this lane's pixel has a winner to shade
-        {
-            const FrameParams &p = args();
-            const View &v = view_of<BATCH>(p, r);
-            const uint32_t mode = key_mode(p);
-            if (ntile != ~0u) ntb = uniform_load(&p.tile_count[ntile]);
-            const uint32_t px = g.X0 + (tid & (g.TW - 1u)), py = g.Y0 + (tid >> sx);
-            if (px < v.W && py < v.H) {
-                const size_t pidx = (size_t)py * v.W + px;
-                const uint64_t kk = sh.key[tid + (tid >> sx)];
-                bool has;  // a winner (its primitive is read again by the shading lanes)
-                float z;
-                if (mode == 0u) {
-                    has = kk != 0ull;
-                    z = __uint_as_float((uint32_t)kk);
-                } else {
-                    has = ((uint32_t)kk) != 0u;
-                    const uint32_t o = (uint32_t)(kk >> 32);
-                    z = zunord(mode == 1u ? o : ~o, (uint32_t)kk & 1u);
-                }
-                shade = v.pixel && p.pixel_write && has && SH != DEPTH_ONLY;
-                if (v.pixel && !shade && v.clear_color_en) store_stream(&v.pixel[pidx], v.clear_color);
-                if (v.depth) {
-                    if (has && p.depth_write) store_stream(&v.depth[pidx], z);
-                    else if (v.clear_depth_en) store_stream(&v.depth[pidx], v.clear_depth);
-                }
-            }
-        }
-        if constexpr (SH != DEPTH_ONLY && (!MS || SH == FLAT)) {  // (FLAT is the same at every coarse sample)
-            // The pixels to shade, packed onto the first lanes in tile order: a wave
-            // with none of them skips the shader.
-            uint32_t total;
-            const uint32_t at = block_rank(sh, tid, shade, total);
-            if (shade) sh.owner[at] = (uint8_t)tid;
-            __syncthreads();
-            if (tid < total) {
+        if (ntile != ~0u) ntb = uniform_load(&args().tile_count[ntile]);
+        // a winner's sample from its setup record and its corners' VertexData
+        resolve_tile<SH, MS>(
+            sh, tid, g, [&]() -> const View & { return view_of<BATCH>(args(), r); },
+            [&](const View &v, uint32_t prim, float X, float Y, float frag[4]) {
                 const FrameParams &p = args();
-                const View &v = view_of<BATCH>(p, r);
-                const uint32_t t = sh.owner[tid];
-                const uint32_t tx2 = g.X0 + (t & (g.TW - 1u)), ty2 = g.Y0 + (t >> sx);
-                const uint32_t prim = key_prim(key_mode(p), sh.key[t + (t >> sx)]) - 1u;
                 TriRec R;
                 load_rec0(p, tri_base + prim, R);
                 tri_sids(v, p.geometry, prim, R.flags, R.sid);
-                float frag[4];
-                shade_sample<SH, GS>(p, v, R, (float)tx2, (float)ty2, frag);
-                store_stream(&v.pixel[(size_t)ty2 * v.W + tx2], blend_shader<SH>(0u, frag, p.bgra));
-            }
-        } else if constexpr (SH != DEPTH_ONLY) {
-            // Coarse shading (pipeline.rs:541-570): a pixel combines four samples of
-            // its winner at the corners of its cell of the band's 2^L grid.  Pixels
-            // of a cell with the same winner have the same samples; a 2 x 2 block
-            // of even band rows and columns always lies in one cell, so the samples
-            // are taken once per block and winner: its first pixel leads.  Each lane
-            // takes one sample of a leader, 64 leaders a round, into LDS, and the
-            // pixels combine them.  (With four samples per pixel and lane the
-            // 1080p terrain's main pass spent three quarters of its vector
-            // instructions on samples that its neighbours took as well.)
-            const uint32_t mode = key_mode(args());
-            const uint32_t tx = tid & (g.TW - 1u), ty = tid >> sx;
-            const uint32_t by0 = sh.band[2 * ty], pid = shade ? key_prim(mode, sh.key[tid + ty]) : 0u;
-            uint32_t leader = tid;
-            if (shade) {
-                const uint32_t odd = (g.Y0 + ty - by0) & 1u;  // second row of its block
-                const uint32_t x0 = tx & ~1u, row = odd ? ty - 1u : ty;
-                const bool above = odd && ty > 0u;  // its first row is in this tile (and then in this band)
-                if (tx & 1u && key_prim(mode, sh.key[ty * (g.TW + 1u) + x0]) == pid) leader = (ty << sx) + x0;
-                if (above) {
-                    if (key_prim(mode, sh.key[row * (g.TW + 1u) + x0 + 1u]) == pid) leader = (row << sx) + x0 + 1u;
-                    if (key_prim(mode, sh.key[row * (g.TW + 1u) + x0]) == pid) leader = (row << sx) + x0;
-                }
-            }
-            uint32_t total;
-            const uint32_t at = block_rank(sh, tid, shade && leader == tid, total);
-            if (shade && leader == tid) sh.owner[at] = (uint8_t)tid, sh.rows_incl[tid] = at;
-            __syncthreads();
-            const uint32_t mine = shade ? sh.rows_incl[leader] : ~0u;  // the leader's rank
-            float4 *const sample = reinterpret_cast<float4 *>(sh.tri);
-            static_assert(sizeof(sh.tri) >= 256u * sizeof(float4), "a round's samples fit the staging space");
-            for (uint32_t b = 0; b < total; b += 64u) {
-                const FrameParams &p = args();
-                const View &v = view_of<BATCH>(p, r);
-                const uint32_t L = p.msaa_level;
-                if (b + (tid >> 2) < total) {
-                    const uint32_t t = sh.owner[b + (tid >> 2)], q = tid & 3u;
-                    const uint32_t prim = key_prim(mode, sh.key[t + (t >> sx)]) - 1u;
-                    const uint32_t b0 = sh.band[2 * (t >> sx)];
-                    const uint32_t cx = (g.X0 + (t & (g.TW - 1u))) >> L, cy = (g.Y0 + (t >> sx) - b0) >> L;
-                    TriRec R;
-                    load_rec0(p, tri_base + prim, R);
-                    tri_sids(v, p.geometry, prim, R.flags, R.sid);
-                    float frag[4];
-                    shade_sample<SH, GS>(p, v, R, (float)((cx + (q & 1u)) << L), (float)(b0 + ((cy + (q >> 1)) << L)), frag);
-                    sample[tid] = make_float4(frag[0], frag[1], frag[2], frag[3]);
-                }
-                __syncthreads();
-                if (mine - b < 64u) {
-                    // bilinear reconstruction (pipeline.rs:556-570)
-                    const float div = 1.0f / (float)(1u << L);
-                    const float fx = rfract((float)(g.X0 + tx) * div), fy = rfract((float)(g.Y0 + ty - by0) * div);
-                    const float4 *s4 = sample + 4u * (mine - b);  // t00, t10, t01, t11
-                    const float4 t00 = s4[0], t10 = s4[1], t01 = s4[2], t11 = s4[3];
-                    const float c00[4] = {t00.x, t00.y, t00.z, t00.w}, c10[4] = {t10.x, t10.y, t10.z, t10.w};
-                    const float c01[4] = {t01.x, t01.y, t01.z, t01.w}, c11[4] = {t11.x, t11.y, t11.z, t11.w};
-                    float frag[4];
+                constexpr uint32_t NV = VDN<SH>::N;
+                float V[3][NV];
 #pragma unroll
-                    for (int c = 0; c < 4; c++) {
-                        const float t0 = c00[c] * (1.0f - fy) + c01[c] * fy;
-                        const float t1 = c10[c] * (1.0f - fy) + c11[c] * fy;
-                        frag[c] = t0 * (1.0f - fx) + t1 * fx;
-                    }
-                    store_stream(&v.pixel[(size_t)(g.Y0 + ty) * v.W + g.X0 + tx], blend_shader<SH>(0u, frag, p.bgra));
+                for (int i = 0; i < 3; i++) {
+                    const float *src = p.vary + (size_t)R.sid[i] * vd_count(SH);
+#pragma unroll
+                    for (uint32_t c = 0; c < vd_count(SH); c++) V[i][c] = src[c];
                 }
-                __syncthreads();  // the next round's samples reuse the space
-            }
-        }
+                shade_sample<SH, GS>(p, v, R, V, X, Y, frag);
+            });
         __syncthreads();
     };
 
@@ -1581,6 +1606,85 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         else if (ntile != ~0u)  // a heavy tile of the busy list: another workgroup's
             ntb = uniform_load(&args().tile_count[ntile]);
         tile = ntile, tb = ntb;
+    }
+}
+
+// k_tiny: one-request frames of few triangles (the rule and both sides' times are
+// at kTinyTris) in one launch.  Every workgroup sets all triangles up itself
+// (a lane each) and computes their corners' VertexData, all kept in LDS, then
+// takes tile after tile: rows of every triangle that reaches into the tile,
+// walked from their starts, and the resolve.  Nothing passes through memory but
+// the mesh, the textures and the targets, and no launch waits for another.  (The
+// walks from the row starts grow with the square of the width, a checkpoint
+// frame's with the width.)
+template <uint32_t SH, bool GS, bool MS>
+__global__ __launch_bounds__(256) void k_tiny(FrameParams) {
+    __shared__ TileShared sh;
+    __shared__ float vd[kTinyTris][3][VDN<SH>::N];
+    warm_args();
+    const uint32_t tid = threadIdx.x;
+    {
+        const FrameParams &p = args();
+        const View &v = p.v0;
+        if (tid < kTinyTris) {
+            TriRec R;
+            R.flags = 0u;
+            const bool keep = tid < v.n_tris && tri_setup(p, v, tid, R);
+            if (!keep) R.ymin = R.ymax = 0u;  // no row in any tile
+            put_tri(sh.tri[tid], R, tid);
+        }
+        __syncthreads();
+        if (tid < 3u * v.n_tris) {  // corner i of triangle t in the order after the winding swap
+            const uint32_t t = tid / 3u, i = tid - 3u * t, c = (sh.tri[t].flags & TRI_SWAPPED) && i != 1u ? 2u - i : i;
+            uint32_t inst[3], at[3];
+            corner_places(v, p.geometry, t, inst, at);
+            const uint32_t in = c == 0u ? inst[0] : c == 1u ? inst[1] : inst[2];
+            const uint32_t k = c == 0u ? at[0] : c == 1u ? at[1] : at[2];
+            vertex_data<SH>(p, v, in, v.idx ? v.idx[k] : k, vd[t][i]);
+        }
+    }
+    for (uint32_t tile = blockIdx.x; tile < args().ntiles; tile += gridDim.x) {
+        TileGeom g;
+        uint32_t rows = 0u;
+        {
+            const FrameParams &p = args();
+            const View &v = p.v0;
+            const uint32_t ty = divide(tile, v.row_tiles), tx = tile - ty * v.ntx;
+            g.sx = p.tile_sx, g.TW = 1u << g.sx, g.TH = 256u >> g.sx;
+            g.X0 = tx << g.sx, g.Y0 = ty << (8u - g.sx);
+            const uint32_t px = g.X0 + (tid & (g.TW - 1u)), py = g.Y0 + (tid >> g.sx);
+            float D0 = 0.0f;
+            if (p.depth_test != DT_NONE || p.depth_write) {
+                D0 = v.clear_depth;
+                if (!v.clear_depth_en && px < v.W && py < v.H) D0 = v.depth[(size_t)py * v.W + px];
+            }
+            const uint32_t lp = tid + (tid >> g.sx);
+            sh.key[lp] = init_key(key_mode(p), D0);
+            sh.d0s[lp] = D0;
+            if (tid < g.TH) {
+                uint32_t by0, by1;
+                band_of(p, v, g.Y0 + tid, by0, by1);
+                sh.band[2 * tid] = by0;
+                sh.band[2 * tid + 1] = by1;
+            }
+            if (tid < v.n_tris) {
+                const TriLds &T = sh.tri[tid];
+                const uint32_t ry0 = T.ymin > g.Y0 ? T.ymin : g.Y0, ry1 = T.ymax < g.Y0 + g.TH ? T.ymax : g.Y0 + g.TH;
+                const bool in = ry0 < ry1 && T.xmin < g.X0 + g.TW && T.xmax > g.X0;
+                rows = in ? ry1 - ry0 : 0u;
+            }
+        }
+        walk_rows<true, true>(sh, tid, rows, g);
+        resolve_tile<SH, MS>(
+            sh, tid, g, [&]() -> const View & { return args().v0; },
+            [&](const View &v, uint32_t prim, float X, float Y, float frag[4]) {
+                const TriLds &T = sh.tri[prim];
+                TriRec R;
+#pragma unroll
+                for (int i = 0; i < 3; i++) R.o[i] = T.o[i], R.dx[i] = T.dx[i], R.dy[i] = T.dy[i];
+                shade_sample<SH, GS>(args(), v, R, vd[prim], X, Y, frag);
+            });
+        __syncthreads();  // the next tile reuses the keys
     }
 }
 
@@ -1662,6 +1766,12 @@ static void launch_raster_g(const FrameParams &p, hipStream_t s, bool batched, u
     else launch_raster_m<SH, GS, false>(p, s, batched, groups);
 }
 
+template <uint32_t SH, bool GS>
+static void launch_tiny_g(const FrameParams &p, hipStream_t s, uint32_t groups) {
+    if (p.msaa_level) hipLaunchKernelGGL((k_tiny<SH, GS, true>), dim3(groups), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((k_tiny<SH, GS, false>), dim3(groups), dim3(256), 0, s, p);
+}
+
 // Textured shaders whose sampler is not their own take the kernels that read
 // textures through any sampler kind.
 template <uint32_t SH>
@@ -1674,6 +1784,18 @@ static void launch_raster_t(const FrameParams &p, hipStream_t s, bool batched, u
         }
     }
     launch_raster_g<SH, false>(p, s, batched, groups);
+}
+
+template <uint32_t SH>
+static void launch_tiny_t(const FrameParams &p, hipStream_t s, uint32_t groups) {
+    if constexpr (SH == TEXTURED || SH == TEX_SHADOW) {
+        const uint32_t own = SH == TEX_SHADOW ? (uint32_t)SAMPLER_LINEAR_CLAMPED : (uint32_t)SAMPLER_LINEAR;
+        if (p.sampler != own) {
+            launch_tiny_g<SH, true>(p, s, groups);
+            return;
+        }
+    }
+    launch_tiny_g<SH, false>(p, s, groups);
 }
 
 // ---------------------------------------------------------------------------
@@ -1884,6 +2006,23 @@ hipError_t launch_raster(const FrameParams &p, hipStream_t s, bool batched) {
     return hipGetLastError();
 }
 
+
+hipError_t launch_tiny(const FrameParams &p, hipStream_t s) {
+    if (p.ntiles == 0) return hipSuccess;
+    const uint32_t g = std::min(p.ntiles, kTinyGroups);
+    switch (p.shader) {
+    case FLAT: launch_tiny_t<FLAT>(p, s, g); break;
+    case COLOR: launch_tiny_t<COLOR>(p, s, g); break;
+    case GOURAUD: launch_tiny_t<GOURAUD>(p, s, g); break;
+    case PHONG: launch_tiny_t<PHONG>(p, s, g); break;
+    case DEPTH_ONLY: launch_tiny_t<DEPTH_ONLY>(p, s, g); break;
+    case TEXTURED: launch_tiny_t<TEXTURED>(p, s, g); break;
+    case PHONG_SHADOW: launch_tiny_t<PHONG_SHADOW>(p, s, g); break;
+    case TEX_SHADOW: launch_tiny_t<TEX_SHADOW>(p, s, g); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
 
 // ---------------------------------------------------------------------------
 // lines (lines.rs:15-121): one-request frames of LineList / LineTriangleList

@@ -564,6 +564,15 @@ euchip_status render_impl(euchip_ctx *ctx, const euchip_pipeline_desc *d, const 
     p.tile_sx = 5;
     p.v0 = P.v;
     tile_grid(p.v0, p.tile_sx);
+    p.ntiles = p.v0.ntx * p.v0.nty;
+    if (P.n_tris <= kTinyTris && P.v.W <= kTinyWidth && P.n_tris * P.v.W * P.v.W <= kTinyWork) {
+        p.n_views = 1;
+        if ((s = timed(ctx, "tiny", [&] { return launch_tiny(p, ctx->stream); }))) return s;
+        if (!sync) return EUCHIP_OK;
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        if (ctx->profiling) resolve_pending(ctx);
+        return EUCHIP_OK;
+    }
     // big-triangle mode when the mesh has no more triangles than the target has
     // 32 x 8 tiles (triangles then tend to cover many tiles each); its tiles are
     // wider (fewer tiles per row walk the same row start)
