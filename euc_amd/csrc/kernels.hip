@@ -1517,41 +1517,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             run = nb + (ckp ? 0u : nbig);  // entries of the current run
         }
         __syncthreads();
-        // Runs of entries, kBatch at a time: this tile's bin and the big
-        // triangles (staging drops those that miss it), then (only when it
-        // overflowed) its overflow segments.  Segments were taken from the pool
-        // in this frame, each pointing at the one taken before it; a walk of at
-        // most pool_used / 3 segments whose every read stays below pool_used
-        // ends even on a damaged list.  One loop, so one copy of raster_batch.
-        uint32_t base = 0u;                 // pool index of the current segment's entries (0: bin + big)
-        uint32_t guard = 0u;
-        for (uint32_t b = 0;; b += kBatch) {
-            while (b >= run) {              // next segment (uniform)
-                if (!seg || guard++ > pool_used / 3u || seg + 1u > pool_used) {
-                    seg = 0u;
-                    break;
-                }
-                const uint32_t *pool = args().pool;
-                const uint32_t s0 = seg - 1u;
-                seg = __builtin_amdgcn_readfirstlane(pool[s0]);
-                const uint32_t len = __builtin_amdgcn_readfirstlane(pool[s0 + 1u]);
-                base = s0 + 2u;
-                run = len < pool_used - base ? len : pool_used - base;
-                b = 0u;
-            }
-            if (b >= run) break;
-            const uint32_t i = b + tid;
+        // Steps of up to kBatch entries: this tile's bin and the big triangles
+        // (staging drops those that miss it), then (only when it overflowed) its
+        // overflow segments, as many as fill a step together.  Segments were taken
+        // from the pool in this frame, each pointing at the one taken before it; a
+        // walk of at most pool_used / 3 segments whose every read stays below
+        // pool_used ends even on a damaged list.  (There is one segment per setup
+        // workgroup that passed the capacity, so often of a few entries: with a
+        // step each, a tile of 831 entries ended a batch's launch 110 us after all
+        // others.)  One loop, so one copy of raster_batch.
+        uint32_t sbase = 0u, slen = 0u, guard = 0u;  // rest of the current segment
+        for (uint32_t b = 0;;) {
             bool valid = false;
             uint32_t prim = 0;
-            if (tid >= kBatch || i >= run) {
-            } else if (base) {
+            if (b < run) {
+                const uint32_t i = b + tid;
+                if (tid >= kBatch || i >= run) {
+                } else if (i < nb) {
+                    valid = true, prim = ahead;
+                    if (i + kBatch < nb) ahead = args().bins[bin_at + i + kBatch];
+                } else if constexpr (BIG) {
+                    valid = true, prim = args().big[i - nb];
+                }
+                b += kBatch;
+            } else {
+                if ((seg | slen) == 0u) break;
+                const uint32_t *pool = args().pool;
+                uint32_t fill = 0u, at = 0u;
+                while (fill < kBatch) {  // uniform
+                    if (slen == 0u) {
+                        if (!seg || guard++ > pool_used / 3u || seg + 1u > pool_used) break;
+                        const uint32_t s0 = seg - 1u;
+                        seg = uniform_load(pool + s0);
+                        slen = uniform_load(pool + s0 + 1u);
+                        sbase = s0 + 2u;
+                        slen = slen < pool_used - sbase ? slen : pool_used - sbase;
+                        continue;
+                    }
+                    const uint32_t take = slen < kBatch - fill ? slen : kBatch - fill;
+                    if (tid - fill < take) at = sbase + (tid - fill);
+                    fill += take, sbase += take, slen -= take;
+                }
+                if (fill == 0u) break;
                 // (read once; a plain load would be merged with the bin's into one FLAT load)
-                valid = true, prim = __builtin_nontemporal_load(&args().pool[base + i]);
-            } else if (i < nb) {
-                valid = true, prim = ahead;
-                if (i + kBatch < nb) ahead = args().bins[bin_at + i + kBatch];
-            } else if constexpr (BIG) {
-                valid = true, prim = args().big[i - nb];
+                valid = tid < fill;
+                if (valid) prim = __builtin_nontemporal_load(&pool[at]);
             }
             raster_batch<!BATCH, BIG>(tri_base, sh, tid, valid, prim, g);
         }
