@@ -518,14 +518,15 @@ euchip_status render_lines(euchip_ctx *ctx, const euchip_pipeline_desc *d, const
     if ((s = ensure(ctx, ctx->lrec, std::max<size_t>((size_t)p.n_lines * kLineRecQuads, 1), "line records",
                     ctx->stream)))
         return s;
-    const uint64_t *keys_had = ctx->lkey.ptr;
+    const size_t keys_had = ctx->lkey.cap;
     if ((s = ensure(ctx, ctx->lkey, npx, "line keys", ctx->stream))) {
         ctx->lkey_clean = false;  // (the old storage is gone)
         return s;
     }
     // new storage starts at zero, as every frame leaves it; after a frame that
-    // was not enqueued whole it starts over
-    if (ctx->lkey.ptr != keys_had) ctx->lkey_clean = false;
+    // was not enqueued whole it starts over (new storage is larger; its address
+    // may be the old one's, freed first to stay within the budget)
+    if (ctx->lkey.cap != keys_had) ctx->lkey_clean = false;
     if (!ctx->lkey_clean)
         HIP_TRY(ctx, launch_fill_u32((uint32_t *)ctx->lkey.ptr, 0u, 2 * ctx->lkey.cap, ctx->stream));
     ctx->lkey_clean = false;

@@ -10,6 +10,7 @@ import pytest
 from euc_amd import scenes as S
 from euc_amd.pipeline import BandPolicy, DepthMode, PipelineDesc, Primitives, Shader, Xform
 from euc_amd.renderer import Context
+from oracle import oracle as O
 from tests.parity import assert_bit_exact, run_pair
 
 pytestmark = pytest.mark.gpu
@@ -54,5 +55,27 @@ def test_keys_between_frames():
             r = run_pair(ctx, desc(dm), S.uniforms(), mesh, w, h, color_init=c, depth_init=z)
             assert r["frags"] > 50
             assert_bit_exact(r, f"frame {k} {dm}")
+    finally:
+        ctx.close()
+
+
+def test_keys_replaced_within_a_budget():
+    """Larger keys that fit the budget only once the old ones are freed (the new
+    storage may then have the old address) start at zero as well."""
+    ctx = Context(0)
+    try:
+        gm = ctx.mesh(lines(7, 300, 40, 640))
+        sizes = [(100, 80), (320, 240), (640, 480)]
+        targets = [(ctx.color_target(*s), ctx.depth_target(*s)) for s in sizes]
+        for k, ((w, h), (c, z)) in enumerate(zip(sizes, targets)):
+            if k:
+                old = sizes[k - 1][0] * sizes[k - 1][1]
+                ctx.set_budget(ctx.bytes_in_use() + 8 * (max(w * h, old + old // 2) - old))
+            ctx.render(desc(DepthMode.LESS_WRITE), S.uniforms(), gm, c, z, clear_color=9, clear_depth=1.0)
+            oc, od = np.full((h, w), 9, np.uint32), np.full((h, w), 1.0, np.float32)
+            rc, frags = O.render(desc(DepthMode.LESS_WRITE), S.uniforms(), lines(7, 300, 40, 640), oc, od)
+            assert rc == 0 and frags > 50
+            assert np.array_equal(c.download(), oc), k
+            assert np.array_equal(z.download().view(np.uint32), od.view(np.uint32)), k
     finally:
         ctx.close()
