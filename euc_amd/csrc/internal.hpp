@@ -123,11 +123,11 @@ enum BusyMap : uint32_t { BUSY_RANGES = 0, BUSY_BLOCKS = 1 };
 constexpr uint32_t kBigTiles = 64;
 constexpr uint32_t kBigCap = 4096;
 
-// One-request frames of few triangles on targets that are not too wide take one
-// launch (k_tiny) of at most kTinyGroups workgroups, no scratch memory and no
-// frame number: at most kTinyTris triangles, kTinyWidth columns, and triangles x
-// columns^2 (what walking every row from its start costs per row) at most
-// kTinyWork.  Against a checkpoint frame, us per pass: a cube of 12 triangles 36.0 /
+// One-request frames of few triangles on targets that are not too wide, of a
+// context without a budget, take one launch (k_tiny) of at most kTinyGroups
+// workgroups, no scratch memory and no frame number: at most kTinyTris triangles,
+// kTinyWidth columns, and triangles x columns^2 (what walking every row from its
+// start costs per row) at most kTinyWork.  Against a checkpoint frame, us per pass: a cube of 12 triangles 36.0 /
 // 26.3 at 800 columns, 60.8 / 38.8 at 1600 (135 / 95 at 3200, but not where
 // triangles fill the target); triangles that each fill it, the worst case: 16 of
 // them 26 / 17 at 640 columns and 50 / 48 at 1280, 64 of them 31 / 32 at 640 and 55
@@ -303,7 +303,7 @@ struct FrameParams {
     uint32_t tri_block, tri_blocks, setup_blocks, span_parts;
     gptr<TileBin> count_next;
     uint32_t zero_n;
-    uint32_t frame;        // frame parity selects the overflow counter and tile queue
+    uint32_t frame;        // frame parity selects the counters
     uint32_t ntiles;       // tiles of all requests
     uint32_t tile_sx;      // tiles are (1 << tile_sx) x (256 >> tile_sx) pixels, tile_sx in 3..5
     // requests: one in `v0` (kernel argument), or `n_views` in device memory

@@ -566,7 +566,10 @@ euchip_status render_impl(euchip_ctx *ctx, const euchip_pipeline_desc *d, const 
     p.v0 = P.v;
     tile_grid(p.v0, p.tile_sx);
     p.ntiles = p.v0.ntx * p.v0.nty;
-    if (P.n_tris <= kTinyTris && P.v.W <= kTinyWidth && P.n_tris * P.v.W * P.v.W <= kTinyWork) {
+    // (a context with a budget keeps to the frames with scratch memory, which
+    // the budget admits or refuses)
+    if (!ctx->budget && P.n_tris <= kTinyTris && P.v.W <= kTinyWidth &&
+        P.n_tris * P.v.W * P.v.W <= kTinyWork) {
         p.n_views = 1;
         if ((s = timed(ctx, "tiny", [&] { return launch_tiny(p, ctx->stream); }))) return s;
         if (!sync) return EUCHIP_OK;

@@ -97,3 +97,25 @@ def test_partial_triangles_and_async(gpu_ctx):
     for k, (c, z, want) in enumerate(outs):
         assert np.array_equal(c.download(), want["o_color"]), k
         assert np.array_equal(z.download().view(np.uint32), want["o_depth"].view(np.uint32)), k
+
+
+def test_budget_refuses_as_before():
+    """A budget that cannot hold the scratch of a binned frame refuses a frame of few triangles too."""
+    from euc_amd._lib import EuchipError
+    from euc_amd.renderer import Context
+    ctx = Context(0)
+    try:
+        m = cube()
+        u = S.uniforms(view_proj=S.f32(S.perspective_fov_lh_zo(1.2, 160, 90, 0.1, 50.0)))
+        d = PipelineDesc.make(Shader.PHONG, Xform.MVP, depth_mode=DepthMode.LESS_WRITE, cull=CullMode.BACK,
+                              band_policy=BandPolicy.SEQ)
+        gm, c, z = ctx.mesh(m), ctx.color_target(160, 90), ctx.depth_target(160, 90)
+        ctx.set_budget(ctx.bytes_in_use())
+        with pytest.raises(EuchipError) as e:
+            ctx.render(d, u, gm, c, z, clear_color=3, clear_depth=1.0)
+        assert e.value.name == "OVER_BUDGET"
+        ctx.set_budget(ctx.bytes_in_use() + (1 << 30))
+        r = run_pair(ctx, d, u, m, 160, 90, color_init=3)
+        assert_bit_exact(r, "within the budget")
+    finally:
+        ctx.close()
