@@ -527,15 +527,21 @@ euchip_status render_lines(euchip_ctx *ctx, const euchip_pipeline_desc *d, const
     // was not enqueued whole it starts over (new storage is larger; its address
     // may be the old one's, freed first to stay within the budget)
     if (ctx->lkey.cap != keys_had) ctx->lkey_clean = false;
-    if (!ctx->lkey_clean)
+    bool clean = true;
+    if (!ctx->lkey_clean) {
         HIP_TRY(ctx, launch_fill_u32((uint32_t *)ctx->lkey.ptr, 0u, 2 * ctx->lkey.cap, ctx->stream));
+        // a fill that is only recorded leaves the keys as they are
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(ctx, hipStreamIsCapturing(ctx->stream, &cap));
+        clean = cap == hipStreamCaptureStatusNone;
+    }
     ctx->lkey_clean = false;
     p.v0.row_pixels = make_divisor(P.v.W);
     p.vary = ctx->vary.ptr;
     p.lrec = ctx->lrec.ptr;
     p.lkey = ctx->lkey.ptr;
     if ((s = timed(ctx, "lines", [&] { return launch_lines(p, ctx->stream); }))) return s;
-    ctx->lkey_clean = true;
+    ctx->lkey_clean = clean;
     if (sync) {
         HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
         if (ctx->profiling) resolve_pending(ctx);

@@ -4,6 +4,8 @@ longer, and with ends thousands of pixels outside (64-bit steps), line counts
 around a workgroup's 16; and frames of other depth modes, sizes and loaded
 targets after one another on one context, which find the keys of the last frame
 zeroed."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -77,5 +79,51 @@ def test_keys_replaced_within_a_budget():
             assert rc == 0 and frags > 50
             assert np.array_equal(c.download(), oc), k
             assert np.array_equal(z.download().view(np.uint32), od.view(np.uint32)), k
+    finally:
+        ctx.close()
+
+
+def test_first_frame_captured():
+    """A context's first lines frame recorded into a graph: the eager frames before
+    and between its replays, and each replay, find the keys zeroed."""
+    hip = C.CDLL("libamdhip64.so.7")
+    w, h = 640, 480
+    ctx = Context(0)
+    old = ctx.color_target(w, 2 * h)  # its storage, all ones, may become the keys
+    old.clear(0xFFFFFFFF)
+    ctx.synchronize()
+    old.close()
+    try:
+        mesh = lines(8, 400, 50, w)
+        gm, stream = ctx.mesh(mesh), C.c_void_p(ctx.stream())
+        d = desc(DepthMode.LESS_WRITE)
+        oc, od = np.full((h, w), 9, np.uint32), np.full((h, w), 1.0, np.float32)
+        rc, frags = O.render(d, S.uniforms(), mesh, oc, od)
+        assert rc == 0 and frags > 50
+        (gc, gz), (ec, ez) = [(ctx.color_target(w, h), ctx.depth_target(w, h)) for _ in range(2)]
+
+        def render(c, z):
+            ctx.render(d, S.uniforms(), gm, c, z, clear_color=9, clear_depth=1.0, sync=False)
+
+        def check(c, z, what):
+            ctx.synchronize()
+            assert np.array_equal(c.download(), oc), what
+            assert np.array_equal(z.download().view(np.uint32), od.view(np.uint32)), what
+
+        graph, ex = C.c_void_p(), C.c_void_p()
+        assert hip.hipStreamBeginCapture(stream, 2) == 0  # relaxed: the frame allocates
+        render(gc, gz)
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+        for k in range(3):
+            render(ec, ez)
+            check(ec, ez, f"eager {k}")
+            ec.clear(0)
+            gc.clear(0)
+            gz.clear(0)
+            assert hip.hipGraphLaunch(ex, stream) == 0
+            check(gc, gz, f"replay {k}")
+        hip.hipGraphExecDestroy(ex)
+        hip.hipGraphDestroy(graph)
     finally:
         ctx.close()
