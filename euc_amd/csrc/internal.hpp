@@ -1,5 +1,7 @@
 // internal.hpp -- structures shared by the host runtime and the gfx950 kernels.
 #pragma once
+#include <algorithm>
+
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -107,6 +109,15 @@ constexpr uint32_t kBatch = 128;
 // Tiles whose bin reaches this many entries are listed by setup and rasterised
 // first (the longest tiles start early instead of ending the launch late).
 constexpr uint32_t kHeavyTile = 128u;
+// Raster workgroups that take the heavy tiles of a frame of n_tris triangles, a
+// multiple of the 8 XCDs: workgroup b reads place b of the list before it knows
+// the list's length, so never more than the list has places.  (The heavy tiles
+// are about the binned triangles / kHeavyTile at most; where there are more, each
+// workgroup takes several.)
+inline uint32_t heavy_group_count(uint32_t heavy_cap, uint32_t n_tris) {
+    const uint32_t want = std::min(512u, n_tris / kHeavyTile / 8u * 8u + 8u);
+    return std::min(want, heavy_cap / 8u * 8u);
+}
 // Which of the 8 busy-tile lists (one per XCD) a tile goes to: its XCD's
 // contiguous tile range (batches: each XCD gets whole requests), or its block
 // of 4 x 4 tiles dealt over the XCDs (one-request frames: each XCD gets a share

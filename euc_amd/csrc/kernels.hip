@@ -1999,9 +1999,8 @@ constexpr uint32_t kFrameGroups = 8192, kBatchGroups = 16384;
 hipError_t launch_raster(const FrameParams &p, hipStream_t s, bool batched) {
     if (p.ntiles == 0) return hipSuccess;
     FrameParams q = p;
-    // (a frame's heavy tiles are about its binned triangles / kHeavyTile at most;
-    // where there are more, each of these workgroups takes several)
-    q.heavy_groups = batched || !p.heavy_cap ? 0u : std::min(512u, std::min(p.heavy_cap, p.v0.n_tris / kHeavyTile) / 8u * 8u + 8u);
+    q.heavy_groups = batched ? 0u : heavy_group_count(p.heavy_cap, p.v0.n_tris);
+    if (!q.heavy_groups) q.heavy_cap = 0u;  // the busy lists' workgroups take every tile
     const uint32_t g = q.heavy_groups + std::min(batched ? kBatchGroups : kFrameGroups, (uint32_t)(((uint64_t)p.ntiles + 7u) / 8u * 8u));
     switch (p.shader) {
     case FLAT: launch_raster_t<FLAT>(q, s, batched, g); break;
