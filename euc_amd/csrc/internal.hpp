@@ -267,6 +267,7 @@ struct FrameParams {
     // per line what its pixels' shading reads, per target pixel a 64-bit winner
     // key, zero between frames
     uint32_t primitives, n_lines;
+    uint32_t line_first;   // the launch's first line
     gptr<uint4> lrec;
     gptr<uint64_t> lkey;
     // per-launch scratch (device)
@@ -369,5 +370,33 @@ enum Prims : uint32_t { PRIMS_TRIANGLES = 0, PRIMS_LINE_LIST = 1, PRIMS_LINE_TRI
 // Line endpoints further than this from the origin (pixels) are not drawn.
 constexpr int32_t kLineCoordLimit = 1 << 29;
 constexpr uint32_t kLineRecQuads = 2;
+
+// A launch has less than 2^32 threads; of longer work each launch takes at most
+// this many workgroups of 256 threads (2^31 threads).
+constexpr uint32_t kLaunchGroups = 1u << 23;
+inline uint32_t launch_groups(uint64_t n, uint32_t per_group) {
+    return (uint32_t)std::min<uint64_t>((n + per_group - 1u) / per_group, kLaunchGroups);
+}
+
+// The launches that draw a frame's lines: each takes the lines from `first` on,
+// kLinesPerBlock a workgroup, the first also the vertices that fit beside them
+// (in one more launch of their own where they do not).
+constexpr uint32_t kLinesPerBlock = 16;
+struct LineLaunch {
+    uint32_t first, line_groups, vertex_groups;
+};
+template <class F>  // f(LineLaunch) per launch
+inline void line_launches(uint32_t n_lines, uint64_t n_vertices, F f) {
+    const uint64_t vg = (n_vertices + 255u) / 256u;
+    const bool beside = vg < kLaunchGroups;
+    if (!beside) f(LineLaunch{0u, 0u, (uint32_t)vg});
+    uint64_t first = 0;
+    do {
+        const LineLaunch q{(uint32_t)first, launch_groups(n_lines - first, kLinesPerBlock),
+                           first == 0 && beside ? (uint32_t)vg : 0u};
+        if (q.line_groups + q.vertex_groups) f(q);
+        first += (uint64_t)q.line_groups * kLinesPerBlock;
+    } while (first < n_lines);
+}
 
 }  // namespace euchip

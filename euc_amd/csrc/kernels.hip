@@ -2129,7 +2129,6 @@ EUCHIP_DEV void walk_line(const FrameParams &p, const View &v, uint32_t l, const
 // between frames: the resolve puts back the ones it finds, so no pass initialises
 // them.  (A launch for the setup, one for the keys, a wave per line with 64-bit
 // divisions and the resolve took 23.5 us for 12,288 lines at 1280x720.)
-constexpr uint32_t kLinesPerBlock = 16;
 constexpr int32_t kLongLine = 256;
 
 template <uint32_t SH, bool LOADS>
@@ -2151,7 +2150,7 @@ __global__ __launch_bounds__(256) void k_line_draw(FrameParams) {
         }
         return;
     }
-    const uint32_t l = blockIdx.x * kLinesPerBlock + (tid >> 4);
+    const uint32_t l = p.line_first + blockIdx.x * kLinesPerBlock + (tid >> 4);
     LineWalk W;
     W.klo = 0, W.khi = -1;
     if (l < p.n_lines) {
@@ -2318,14 +2317,17 @@ template <uint32_t SH>
 static void launch_lines_t(const FrameParams &p, hipStream_t s) {
     const size_t nsv = (size_t)p.v0.n_instances * p.v0.n_vertices;
     const size_t npx = (size_t)p.v0.W * p.v0.H;
-    FrameParams q = p;
-    q.tri_blocks = blocks_of(p.n_lines, kLinesPerBlock);
-    const uint32_t blocks = q.tri_blocks + (vd_count(SH) > 0 ? blocks_of(nsv, 256) : 0u);
-    if (p.depth_test != DT_NONE && !p.v0.clear_depth_en)
-        hipLaunchKernelGGL((k_line_draw<SH, true>), dim3(blocks), dim3(256), 0, s, q);
-    else
-        hipLaunchKernelGGL((k_line_draw<SH, false>), dim3(blocks), dim3(256), 0, s, q);
-    hipLaunchKernelGGL((k_line_resolve<SH>), dim3(blocks_of(npx, 256)), dim3(256), 0, s, q);
+    line_launches(p.n_lines, vd_count(SH) > 0 ? nsv : 0u, [&](const LineLaunch &l) {
+        FrameParams q = p;
+        q.line_first = l.first;
+        q.tri_blocks = l.line_groups;
+        const dim3 blocks(l.line_groups + l.vertex_groups);
+        if (p.depth_test != DT_NONE && !p.v0.clear_depth_en)
+            hipLaunchKernelGGL((k_line_draw<SH, true>), blocks, dim3(256), 0, s, q);
+        else
+            hipLaunchKernelGGL((k_line_draw<SH, false>), blocks, dim3(256), 0, s, q);
+    });
+    hipLaunchKernelGGL((k_line_resolve<SH>), dim3(blocks_of(npx, 256)), dim3(256), 0, s, p);
 }
 
 hipError_t launch_lines(const FrameParams &p, hipStream_t s) {
@@ -2345,9 +2347,15 @@ hipError_t launch_lines(const FrameParams &p, hipStream_t s) {
 }
 
 hipError_t launch_fill_u32(uint32_t *dst, uint32_t value, size_t n, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fill_u32, dim3(blocks_of(n, 256)), dim3(256), 0, s, dst, value, n);
-    return hipGetLastError();
+    while (n) {
+        const uint32_t groups = launch_groups(n, 256u);
+        const size_t part = std::min<size_t>(n, (size_t)groups * 256u);
+        hipLaunchKernelGGL(k_fill_u32, dim3(groups), dim3(256), 0, s, dst, value, part);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        dst += part, n -= part;
+    }
+    return hipSuccess;
 }
 
 }  // namespace euchip
