@@ -1051,7 +1051,7 @@ struct TileShared {
     // lanes walking the same column of different rows hit different banks.
     uint64_t key[256 + kMaxTileH];  // winner key
     float d0s[256 + kMaxTileH];     // depth before the pass (the test's reference)
-    TriLds tri[kBatch];             // the batch's triangles
+    alignas(16) TriLds tri[kBatch]; // the batch's triangles (also coarse samples, 16 bytes each)
     uint32_t rows_incl[256];        // inclusive prefix sum of their row counts in the tile
     uint8_t owner[256];             // entry of each (entry, row) item of the current 256
     uint32_t wave_rows[4];          // row counts per wave (prefix-sum carry)
@@ -1319,6 +1319,9 @@ EUCHIP_DEV void resolve_tile(TileShared &sh, uint32_t tid, const TileGeom &g, Vi
         const uint32_t mine = shade ? sh.rows_incl[leader] : ~0u;  // the leader's rank
         float4 *const samples = reinterpret_cast<float4 *>(&sh.tri[kTinyTris]);
         static_assert(sizeof(TriLds) * (kBatch - kTinyTris) >= 256u * sizeof(float4), "a round's samples fit the staging space");
+        static_assert(alignof(TileShared) % alignof(float4) == 0u &&
+                          (offsetof(TileShared, tri) + kTinyTris * sizeof(TriLds)) % alignof(float4) == 0u,
+                      "samples are read and written 16 bytes at a time");
         for (uint32_t b = 0; b < total; b += 64u) {
             const FrameParams &p = args();
             const View &v = view();
