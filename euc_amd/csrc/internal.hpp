@@ -358,8 +358,6 @@ hipError_t launch_setup(const FrameParams &p, hipStream_t s, bool batched, uint3
 hipError_t launch_raster(const FrameParams &p, hipStream_t s, bool batched);
 // The whole frame of a small mesh (p.v0): setup and raster in one launch.
 hipError_t launch_tiny(const FrameParams &p, hipStream_t s);
-// Row checkpoints of the big triangles (one-request big-triangle frames with a
-// checkpoint pool), between setup and raster.
 hipError_t launch_fill_u32(uint32_t *dst, uint32_t value, size_t n, hipStream_t s);
 // The lines path of one request (p.v0): vertex stage beside line setup and walk,
 // then every pixel resolved (colour, depth, clears).

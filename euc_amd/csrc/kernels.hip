@@ -794,22 +794,9 @@ EUCHIP_DEV uint32_t key_prim(uint32_t mode, uint64_t kk) {
     return mode == 0u ? (uint32_t)(kk >> 32) : (uint32_t)kk >> 1;
 }
 
-EUCHIP_DEV void update_key(uint64_t *key, uint32_t mode, uint32_t test, float z, float D0, uint32_t prim) {
-    if (mode == 0u) {
-        bool pass;
-        switch (test) {
-        case DT_LESS: pass = z < D0; break;
-        case DT_EQUAL: pass = z == D0; break;
-        case DT_GREATER: pass = z > D0; break;
-        default: pass = true; break;
-        }
-        if (pass) atomicMax((unsigned long long *)key, ((uint64_t)(prim + 1u) << 32) | __float_as_uint(z));
-    } else {
-        if (z != z) return;
-        const uint32_t o = mode == 1u ? zord(z) : ~zord(z);
-        const uint32_t nz = __float_as_uint(z) == 0x80000000u ? 1u : 0u;
-        atomicMin((unsigned long long *)key, ((uint64_t)o << 32) | ((prim + 1u) << 1) | nz);
-    }
+// The depth test of a pixel whose depth before the pass is D0 (not DT_NONE).
+EUCHIP_DEV bool passes_depth(uint32_t test, float z, float D0) {
+    return test == DT_LESS ? z < D0 : test == DT_EQUAL ? z == D0 : z > D0;
 }
 
 // Row span [x0, x1) of row y for a triangle (triangles.rs:219-254); the
@@ -887,16 +874,16 @@ struct TileGeom {
 
 // The tile's pixels [xs, xe) of one row (LDS index pi0 of the first), w_hom at
 // xs given: each pixel's fragment updates its winner key.  Rows of small
-// triangles in key mode 0 (the test reads the depth before the pass); the
-// write modes take walk_span's loop.
-template <uint32_t MODE>
+// triangles where the test reads the depth before the pass (key mode 0 with a
+// depth test); the others take walk_span's loops.
 EUCHIP_DEV void walk_row(const FrameParams &p, const TriRec &R, uint32_t prim, uint32_t xs, uint32_t xe, uint32_t pi0,
                          float w0, float w1, float w2, uint64_t *key, const float *d0s) {
     for (uint32_t x = xs; x < xe; x++) {
         float z;
         if (frag_z(p, R, w0, w1, w2, z)) {
             const uint32_t pi = pi0 + (x - xs);
-            update_key(key + pi, MODE, p.depth_test, z, MODE == 0u ? d0s[pi] : 0.0f, prim);
+            if (passes_depth(p.depth_test, z, d0s[pi]))
+                atomicMax((unsigned long long *)(key + pi), ((uint64_t)(prim + 1u) << 32) | __float_as_uint(z));
         }
         w0 = w0 + R.dx[0];
         w1 = w1 + R.dx[1];
@@ -989,8 +976,7 @@ EUCHIP_DEV void walk_span(const FrameParams &p, const TriRec &R, uint32_t prim, 
         ok = ok & (!clip | ((zlo <= z) & (z <= zhi)));
         const uint32_t pi = pi0 + (x - xs);
         const float D0 = d0s[pi];
-        const bool pass = test == DT_LESS ? z < D0 : test == DT_EQUAL ? z == D0 : test == DT_GREATER ? z > D0 : true;
-        if (ok & pass) atomicMax((unsigned long long *)(key + pi), ((uint64_t)pid << 32) | __float_as_uint(z));
+        if (ok & passes_depth(test, z, D0)) atomicMax((unsigned long long *)(key + pi), ((uint64_t)pid << 32) | __float_as_uint(z));
         w0 = w0 + R.dx[0];
         w1 = w1 + R.dx[1];
         w2 = w2 + R.dx[2];
@@ -1034,7 +1020,7 @@ EUCHIP_DEV void raster_row(const FrameParams &p, const TriRec &R, uint32_t prim,
     if (mode == 1u) walk_span<1u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
     else if (mode == 2u) walk_span<2u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
     else if (p.depth_test == DT_NONE) walk_span<3u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
-    else walk_row<0u>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
+    else walk_row(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
 }
 
 constexpr uint32_t kMaxTileH = 32;
@@ -2112,7 +2098,7 @@ EUCHIP_DEV void walk_line(const FrameParams &p, const View &v, uint32_t l, const
         const size_t pi = (size_t)y * v.W + x;
         if (p.depth_test != DT_NONE) {
             const float D0 = LOADS ? v.depth[pi] : v.clear_depth;
-            if (!(p.depth_test == DT_LESS ? z < D0 : p.depth_test == DT_EQUAL ? z == D0 : z > D0)) continue;
+            if (!passes_depth(p.depth_test, z, D0)) continue;
         }
         // the keys of init_key, those of the write modes complemented
         uint64_t key = ((uint64_t)(l + 1u) << 32) | __float_as_uint(z);
