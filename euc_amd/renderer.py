@@ -187,8 +187,12 @@ def _requests_c(reqs):
     n = len(reqs)
     if n == 0:
         return (RequestC * 1)()
-    u = np.concatenate([r.uniforms for r in reqs], axis=None, dtype=np.float32)
-    assert u.size == n * N_UNIFORMS
+    us = [r.uniforms for r in reqs]
+    if set(map(len, us)) != {N_UNIFORMS}:  # several dimensions, or replaced by the caller
+        us = [np.asarray(u).reshape(-1)[:N_UNIFORMS] for u in us]
+    u = np.concatenate(us, axis=None, dtype=np.float32)
+    if u.size != n * N_UNIFORMS:
+        raise ValueError(f"a request has fewer than {N_UNIFORMS} uniforms")
     at, ptrs = _address(u), []
     for r in reqs:
         p, d, t, s = r.pixel, r.depth, r.texture, r.shadow
