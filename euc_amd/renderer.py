@@ -345,6 +345,8 @@ class Context:
         _check(self.handle, _lib.lib().euchip_set_profiling(self.handle, int(on)))
 
     def kernel_stats(self) -> dict:
+        """{name: (launches, total ms)} since reset_stats(), while profiling is on
+        (the names are listed at euchip_kernel_stat in include/euchip.h)."""
         L = _lib.lib()
         n = L.euchip_kernel_stats(self.handle, None, 0)
         arr = (KernelStatC * max(n, 1))()

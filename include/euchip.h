@@ -151,7 +151,11 @@ typedef struct euchip_mesh_desc {
 } euchip_mesh_desc;
 
 /* Per-kernel timing collected while profiling is on (hipEvents on the
- * context's stream around each launch). */
+ * context's stream around each launch).  Names: "setup" and "raster", the two
+ * launches of a triangle frame; "tiny", the one launch that does both for a frame
+ * of few triangles (at most 64; such a frame adds nothing to the other two);
+ * "lines", all launches of a lines frame; "batch_setup" and "batch_raster", those
+ * of a batch launched without a graph; "clear", a buffer's clear. */
 typedef struct euchip_kernel_stat {
     char name[32];
     uint64_t launches;
