@@ -111,9 +111,9 @@ constexpr uint32_t kBatch = 128;
 constexpr uint32_t kHeavyTile = 128u;
 // Raster workgroups that take the heavy tiles of a frame of n_tris triangles, a
 // multiple of the 8 XCDs: workgroup b reads place b of the list before it knows
-// the list's length, so never more than the list has places.  (The heavy tiles
-// are about the binned triangles / kHeavyTile at most; where there are more, each
-// workgroup takes several.)
+// the list's length, so never more than the list has places.  (Small triangles
+// make about n_tris / kHeavyTile tiles heavy at most; for frames with more see
+// k_raster.)
 inline uint32_t heavy_group_count(uint32_t heavy_cap, uint32_t n_tris) {
     const uint32_t want = std::min(512u, n_tris / kHeavyTile / 8u * 8u + 8u);
     return std::min(want, heavy_cap / 8u * 8u);

@@ -1357,21 +1357,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
     __shared__ TileShared sh;
     warm_args();
     const uint32_t tid = threadIdx.x;
-    // p.heavy_groups workgroups for the heavy tiles, so that the longest tiles
-    // start first, then one per tile of the launch (see launch_raster): the w-th
-    // of its XCD takes busy tile w of the XCD's list and clears tile t0 + w if it
-    // is empty.  The hardware starts them as others end: a queue of tiles for
-    // resident workgroups took a returning atomic, a list load and a count load
-    // per tile, one after the other, and left the empty tiles to the end.  A
-    // workgroup's own chain of loads is short and all of it scalar: counters, list
-    // entry and counts cost no vector instruction.  Against that queue: a
-    // 1366x768 Gouraud frame 26.7 -> 23.1 us, 1080p Phong 42.8 -> 36.8, 3840x2160
-    // 128 -> 126, a batch of 1024 icons 446 -> 416.
+    // p.heavy_groups workgroups for the heavy tiles, so that the longest tiles start
+    // first, then one per tile of the launch (see launch_raster): the w-th of its XCD
+    // takes busy tile w of the XCD's list and clears tile t0 + w if it is empty.  The
+    // hardware starts them as others end: a queue of tiles for resident workgroups
+    // took a returning atomic, a list load and a count load per tile, one after the
+    // other, and left the empty tiles to the end.  A workgroup's own chain of loads is
+    // short and all of it scalar: counters, list entry and counts cost no vector
+    // instruction.  Against that queue: a 1366x768 Gouraud frame 26.7 -> 23.1 us,
+    // 1080p Phong 42.8 -> 36.8, 3840x2160 128 -> 126, a batch of 1024 icons 446 ->
+    // 416.
+    // Where more tiles are heavy than have a workgroup of their own (large triangles
+    // in many tiles each, dense meshes), all tiles are taken by the workgroups of the
+    // busy lists, none in front, except that twice as many heavy tiles, while they are
+    // an eighth of the frame's tiles at most, go in front still, two to a workgroup.
+    // With all left to the heavy workgroups / as now, us: a 640x480 frame of 3000
+    // large triangles (24 workgroups for 2400 heavy tiles) 2600 / 246, 1280x720 frames
+    // of 1.2 million small ones 279 / 143 and of 590,000 51 / 43.  With none in front
+    // past one each / as now: the 1080p terrain 110.7 / 106.2, a 1080p torus frame of
+    // 590,000 triangles 51.1 / 49.1; without the bound of an eighth that 1280x720
+    // frame takes 50.3.
     const uint32_t xcd = blockIdx.x & 7u;
     uint32_t w, per_xcd, nh, nbusy, nbig, pool_used, tile;
     uint32_t t0, t1;   // the XCD's contiguous range of tiles
     uint32_t count;    // bin entries of tile t0 + w
     bool clears;       // it has such a tile and the frame has clears
+    bool heavy_apart = !BATCH;  // heavy tiles go to the heavy workgroups, not with the busy ones
     {
         const FrameParams &p = args();
         const uint32_t par = p.frame & 1u, npar = (p.frame + 1u) & 1u;
@@ -1423,7 +1434,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
         if (BIG && !p.ck_on) nbig = nbig < p.big_cap ? nbig : p.big_cap;
         nh = nh < p.heavy_cap ? nh : p.heavy_cap;
         nbusy = nbusy < lcap ? nbusy : lcap;
-        if (for_heavy ? blockIdx.x >= nh : false) return;
+        if constexpr (!BATCH) {
+            heavy_apart = p.heavy_cap && (nh <= p.heavy_groups || (nh <= 2u * p.heavy_groups && nh <= p.ntiles / 8u));
+            if (for_heavy && (!heavy_apart || blockIdx.x >= nh)) return;
+        }
         // With big triangles every tile may hold fragments: each workgroup then
         // takes its tile of the XCD's contiguous range, none is cleared apart.
         if (BIG && nbig) nbusy = t1 - t0, clears = false, tile = for_heavy ? tile : t0 + w;
@@ -1601,7 +1615,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_wave
             else ntile = uniform_load(p.busy + lbase + k);
         }
         TileBin ntb{0u, 0u};
-        if (heavy || !args().heavy_cap || tb.count < kHeavyTile)
+        if (heavy || !heavy_apart || tb.count < kHeavyTile)
             run_tile(tile, tb.count, tb.head, ntile, ntb);
         else if (ntile != ~0u)  // a heavy tile of the busy list: another workgroup's
             ntb = uniform_load(&args().tile_count[ntile]);
