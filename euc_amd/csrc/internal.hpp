@@ -377,23 +377,23 @@ inline uint32_t launch_groups(uint64_t n, uint32_t per_group) {
 }
 
 // The launches that draw a frame's lines: each takes the lines from `first` on,
-// kLinesPerBlock a workgroup, the first also the vertices that fit beside them
-// (in one more launch of their own where they do not).
+// per_group a workgroup, the first also the vertices that fit beside them (in one
+// more launch of their own where they do not).
 constexpr uint32_t kLinesPerBlock = 16;
 struct LineLaunch {
     uint32_t first, line_groups, vertex_groups;
 };
 template <class F>  // f(LineLaunch) per launch
-inline void line_launches(uint32_t n_lines, uint64_t n_vertices, F f) {
+inline void line_launches(uint32_t n_lines, uint64_t n_vertices, F f, uint32_t per_group = kLinesPerBlock) {
     const uint64_t vg = (n_vertices + 255u) / 256u;
     const bool beside = vg < kLaunchGroups;
     if (!beside) f(LineLaunch{0u, 0u, (uint32_t)vg});
     uint64_t first = 0;
     do {
-        const LineLaunch q{(uint32_t)first, launch_groups(n_lines - first, kLinesPerBlock),
+        const LineLaunch q{(uint32_t)first, launch_groups(n_lines - first, per_group),
                            first == 0 && beside ? (uint32_t)vg : 0u};
         if (q.line_groups + q.vertex_groups) f(q);
-        first += (uint64_t)q.line_groups * kLinesPerBlock;
+        first += (uint64_t)q.line_groups * per_group;
     } while (first < n_lines);
 }
 

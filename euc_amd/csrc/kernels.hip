@@ -2124,17 +2124,24 @@ EUCHIP_DEV void walk_line(const FrameParams &p, const View &v, uint32_t l, const
     }
 }
 
-// k_line_draw: blocks of 16 lines, then vertex blocks (lane t = shaded vertex t).
-// 16 lanes set a line up (lines.rs:41-86 in f32 over the whole target; the band
-// clamp of the clip rectangle only cuts rows other bands draw), each for itself,
-// and take its steps k, k + 16, ...; lines of more than kLongLine pixels are
-// walked by the whole wave, one after the other.  The per-pixel keys are zero
+// k_line_draw: blocks of 256 / LANES lines, then vertex blocks (lane t = shaded
+// vertex t).  LANES lanes set a line up (lines.rs:41-86 in f32 over the whole
+// target; the band clamp of the clip rectangle only cuts rows other bands draw),
+// each for itself, and take its steps k, k + LANES, ...; with 16, lines of more
+// than kLongLine pixels are walked by the whole wave, one after the other.  The per-pixel keys are zero
 // between frames: the resolve puts back the ones it finds, so no pass initialises
 // them.  (A launch for the setup, one for the keys, a wave per line with 64-bit
 // divisions and the resolve took 23.5 us for 12,288 lines at 1280x720.)
+// Frames of up to kWaveLines lines, whose waves do not fill the chip, give a line
+// a whole wave: four long ones in turn are a serial chain, of loads and atomics
+// where the depth is read.  16 lanes / a wave, us at 1920x1080: 300 lines of 900
+// pixels 32.4 / 18.4, over loaded depth 36.9 / 16.3, 1000 of them 36.6 / 30.5 and
+// 39.9 / 18.1; of 30 pixels, 2000 lines 14.2 / 13.8, 8000 20.0 / 20.3, 20,000 32.2 /
+// 33.8; of 5 pixels, 1000 lines 11.4 / 11.6, 4000 12.7 / 14.0, 12,000 15.2 / 19.8.
 constexpr int32_t kLongLine = 256;
+constexpr uint32_t kWaveLines = 2048;
 
-template <uint32_t SH, bool LOADS>
+template <uint32_t SH, bool LOADS, uint32_t LANES>
 __global__ __launch_bounds__(256) void k_line_draw(FrameParams) {
     warm_args();
     const FrameParams &p = args();
@@ -2153,7 +2160,7 @@ __global__ __launch_bounds__(256) void k_line_draw(FrameParams) {
         }
         return;
     }
-    const uint32_t l = p.line_first + blockIdx.x * kLinesPerBlock + (tid >> 4);
+    const uint32_t l = p.line_first + blockIdx.x * (256u / LANES) + tid / LANES;
     LineWalk W;
     W.klo = 0, W.khi = -1;
     if (l < p.n_lines) {
@@ -2203,11 +2210,15 @@ __global__ __launch_bounds__(256) void k_line_draw(FrameParams) {
             W.klo = klo < 0 ? 0 : klo;
             W.khi = khi > (int32_t)W.dM ? (int32_t)W.dM : khi;
         }
-        if ((tid & 15u) == 0u) {  // what the resolve reads of the line
+        if (tid % LANES == 0u) {  // what the resolve reads of the line
             uint4 *rq = p.lrec + (size_t)l * kLineRecQuads;
             rq[0] = make_uint4(__float_as_uint(W.vs0), __float_as_uint(W.norm), sid[0], sid[1]);
             rq[1] = make_uint4(W.use_x ? 1u : 0u, 0u, 0u, 0u);
         }
+    }
+    if constexpr (LANES == 64u) {
+        walk_line<LOADS>(p, v, l, W, lane_id(), 64u);
+        return;
     }
     const bool wide = W.khi - W.klo >= kLongLine;
     if (!wide) walk_line<LOADS>(p, v, l, W, tid & 15u, 16u);
@@ -2320,16 +2331,18 @@ template <uint32_t SH>
 static void launch_lines_t(const FrameParams &p, hipStream_t s) {
     const size_t nsv = (size_t)p.v0.n_instances * p.v0.n_vertices;
     const size_t npx = (size_t)p.v0.W * p.v0.H;
-    line_launches(p.n_lines, vd_count(SH) > 0 ? nsv : 0u, [&](const LineLaunch &l) {
+    const bool waves = p.n_lines <= kWaveLines, loads = p.depth_test != DT_NONE && !p.v0.clear_depth_en;
+    auto draw = [&](const LineLaunch &l) {
         FrameParams q = p;
         q.line_first = l.first;
         q.tri_blocks = l.line_groups;
         const dim3 blocks(l.line_groups + l.vertex_groups);
-        if (p.depth_test != DT_NONE && !p.v0.clear_depth_en)
-            hipLaunchKernelGGL((k_line_draw<SH, true>), blocks, dim3(256), 0, s, q);
-        else
-            hipLaunchKernelGGL((k_line_draw<SH, false>), blocks, dim3(256), 0, s, q);
-    });
+        if (loads && waves) hipLaunchKernelGGL((k_line_draw<SH, true, 64>), blocks, dim3(256), 0, s, q);
+        else if (loads) hipLaunchKernelGGL((k_line_draw<SH, true, 16>), blocks, dim3(256), 0, s, q);
+        else if (waves) hipLaunchKernelGGL((k_line_draw<SH, false, 64>), blocks, dim3(256), 0, s, q);
+        else hipLaunchKernelGGL((k_line_draw<SH, false, 16>), blocks, dim3(256), 0, s, q);
+    };
+    line_launches(p.n_lines, vd_count(SH) > 0 ? nsv : 0u, draw, waves ? 4u : kLinesPerBlock);
     hipLaunchKernelGGL((k_line_resolve<SH>), dim3(blocks_of(npx, 256)), dim3(256), 0, s, p);
 }
 
