@@ -134,18 +134,29 @@ enum BusyMap : uint32_t { BUSY_RANGES = 0, BUSY_BLOCKS = 1 };
 constexpr uint32_t kBigTiles = 64;
 constexpr uint32_t kBigCap = 4096;
 
-// One-request frames of few triangles on targets that are not too wide, of a
-// context without a budget, take one launch (k_tiny) of at most kTinyGroups
-// workgroups, no scratch memory and no frame number: at most kTinyTris triangles,
-// kTinyWidth columns, and triangles x columns^2 (what walking every row from its
-// start costs per row) at most kTinyWork.  Against a checkpoint frame, us per pass: a cube of 12 triangles 36.0 /
-// 26.3 at 800 columns, 60.8 / 38.8 at 1600 (135 / 95 at 3200, but not where
-// triangles fill the target); triangles that each fill it, the worst case: 16 of
-// them 26 / 17 at 640 columns and 50 / 48 at 1280, 64 of them 31 / 32 at 640 and 55
-// / 113 at 1280, 2 of them 49 / 39 at 1280 and 79 / 91 at 1920.
+// One-request frames of few triangles, of a context without a budget, take one
+// launch (k_tiny) of at most kTinyGroups workgroups, no scratch memory and no
+// frame number, while its row walks cost less than what they save.  Every tile
+// walks its rows of every triangle from their starts, which per pixel grows with
+// triangles x columns; what it saves is a checkpoint frame's fixed cost (6e10 in
+// the units of the walk) and its reads per pixel (8000).  Where the two cross
+// depends on how much of the target the triangles fill, which only the device
+// knows.  The constants are a fit over 967 frames of 1 to 64 triangles, 64 to 3840
+// columns and 50 to 7680 rows, whose triangles each fill the target or span 0.4 of
+// each side.  Checkpoint / tiny frame, us: on the tiny side the smaller triangles
+// gain 1.07 to 2x, those that fill the target up to 1.9x or lose, 0.74x at worst
+// (filling: 12 at 1280x720 48 / 40, 2 at 1920x1080 72 / 47, 64 at 640x400 26 / 30,
+// 20 at 960x2000 60 / 81); on the other side, filling, 12 at 1600x1600 81 / 95, 64 at
+// 640x1920 40 / 76, 64 at 3840x2160 213 / 1773.  A tile of more than 32 triangles
+// takes a second round of rows.  Wider targets gain or lose by the scene, filling:
+// 2 triangles at 2560x700 75 / 86, 4 at 3000x400 77 / 101.
 constexpr uint32_t kTinyTris = 64;
-constexpr uint32_t kTinyWidth = 1600;
-constexpr uint64_t kTinyWork = (uint64_t)12 * 1600 * 1600;
+constexpr uint32_t kTinyWidth = 2048;
+inline bool tiny_frame(uint64_t n_tris, uint32_t W, uint32_t H) {
+    if (n_tris > kTinyTris || W > kTinyWidth) return false;
+    const double walk = (double)(n_tris + 12u + (n_tris > 32u ? 192u : 0u)) * W;
+    return walk <= 8000.0 + 6e10 / ((double)W * H);
+}
 constexpr uint32_t kTinyGroups = 1536;  // what the compute units hold at once (6 each)
 
 // Row checkpoints of big triangles.  The exact walk of a row (w += dx from the

@@ -574,8 +574,7 @@ euchip_status render_impl(euchip_ctx *ctx, const euchip_pipeline_desc *d, const 
     p.ntiles = p.v0.ntx * p.v0.nty;
     // (a context with a budget keeps to the frames with scratch memory, which
     // the budget admits or refuses)
-    if (!ctx->budget && P.n_tris <= kTinyTris && P.v.W <= kTinyWidth &&
-        P.n_tris * P.v.W * P.v.W <= kTinyWork) {
+    if (!ctx->budget && tiny_frame(P.n_tris, P.v.W, P.v.H)) {
         p.n_views = 1;
         if ((s = timed(ctx, "tiny", [&] { return launch_tiny(p, ctx->stream); }))) return s;
         if (!sync) return EUCHIP_OK;
