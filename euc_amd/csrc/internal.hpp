@@ -278,7 +278,6 @@ struct FrameParams {
     // per line what its pixels' shading reads, per target pixel a 64-bit winner
     // key, zero between frames
     uint32_t primitives, n_lines;
-    uint32_t line_first;   // the launch's first line
     gptr<uint4> lrec;
     gptr<uint64_t> lkey;
     // per-launch scratch (device)
@@ -291,6 +290,7 @@ struct FrameParams {
     gptr<uint32_t> req_max;     // batches, per request: largest tile count above its tile_cap (host grows the bins)
     gptr<uint32_t> pool;        // overflow segments (ranks >= tile_cap), pool_cap words
     uint32_t pool_cap;
+    uint32_t line_first;   // the launch's first line
     gptr<Report> report;        // host-visible report of one-request frames, or null
     gptr<uint32_t> heavy;       // tiles with at least kHeavyTile entries (heavy_cap slots)
     uint32_t heavy_cap;    // 0: no heavy-first pass

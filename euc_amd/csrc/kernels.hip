@@ -875,14 +875,17 @@ struct TileGeom {
 // The tile's pixels [xs, xe) of one row (LDS index pi0 of the first), w_hom at
 // xs given: each pixel's fragment updates its winner key.  Rows of small
 // triangles where the test reads the depth before the pass (key mode 0 with a
-// depth test); the others take walk_span's loops.
+// depth test); the others take walk_span's loops.  One loop per test: with the test
+// chosen inside it, a 1280x720 frame of 12 triangles over loaded depth 53.5 us
+// instead of 47.8, one of 6000 large triangles 180 instead of 154.
+template <uint32_t TEST>
 EUCHIP_DEV void walk_row(const FrameParams &p, const TriRec &R, uint32_t prim, uint32_t xs, uint32_t xe, uint32_t pi0,
                          float w0, float w1, float w2, uint64_t *key, const float *d0s) {
     for (uint32_t x = xs; x < xe; x++) {
         float z;
         if (frag_z(p, R, w0, w1, w2, z)) {
             const uint32_t pi = pi0 + (x - xs);
-            if (passes_depth(p.depth_test, z, d0s[pi]))
+            if (passes_depth(TEST, z, d0s[pi]))
                 atomicMax((unsigned long long *)(key + pi), ((uint64_t)(prim + 1u) << 32) | __float_as_uint(z));
         }
         w0 = w0 + R.dx[0];
@@ -1020,7 +1023,9 @@ EUCHIP_DEV void raster_row(const FrameParams &p, const TriRec &R, uint32_t prim,
     if (mode == 1u) walk_span<1u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
     else if (mode == 2u) walk_span<2u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
     else if (p.depth_test == DT_NONE) walk_span<3u, (SKIP_UNROLL > 4u)>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
-    else walk_row(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
+    else if (p.depth_test == DT_LESS) walk_row<DT_LESS>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
+    else if (p.depth_test == DT_EQUAL) walk_row<DT_EQUAL>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
+    else walk_row<DT_GREATER>(p, R, prim, xs, xe, pi0, w0, w1, w2, key, d0s);
 }
 
 constexpr uint32_t kMaxTileH = 32;
