@@ -92,3 +92,26 @@ def test_who_takes_heavy_tiles(gpu_ctx, w, h, n, region, kind):
         r = run_pair(gpu_ctx, DESC, S.uniforms(), mesh, w, h, color_init=rep, gmesh=gm)
         assert_bit_exact(r, f"{kind}, frame {rep}")
     assert r["frags"] > 1000
+
+
+@pytest.mark.parametrize("region,kind", [((0.30, 0.06), "busy"), ((0.16, 0.045), "two"), ((0.06, 0.03), "own")])
+def test_big_triangle_frames(gpu_ctx, region, kind):
+    """The same where a frame also has large triangles that are on no tile's list (no row checkpoints)."""
+    w = h = 2048
+    n, n_large = 16000, 6
+    rng = np.random.default_rng(6)
+    pos = np.ones((n + n_large, 3, 4), np.float32)
+    pos[:n, :, :2] = rng.uniform(-1.0, 1.0, (n, 1, 2)) * region + rng.uniform(-1.0, 1.0, (n, 3, 2)) * [0.016, 0.012]
+    pos[n:, :, :2] = rng.uniform(-1.0, 1.0, (n_large, 3, 2))
+    pos[:, :, 2] = rng.uniform(0.05, 0.95, (n + n_large, 1))
+    mesh = S.Mesh(pos=pos.reshape(-1, 4), count=3 * (n + n_large),
+                  rgba8=rng.integers(0, 2 ** 32, 3 * (n + n_large), dtype=np.uint64).astype(np.uint32))
+    small = S.Mesh(pos=pos[:n].reshape(-1, 4), count=3 * n)
+    groups, tiles, heavy = n // 128 // 8 * 8 + 8, 64 * 256, heavy_tiles(small, w, h)
+    assert n + n_large <= tiles and tiles * n > 8 << 20  # big-triangle mode, without checkpoints
+    assert kind == ("own" if heavy <= groups else "two" if heavy <= 2 * groups else "busy"), (heavy, groups)
+    gm = gpu_ctx.mesh(mesh)
+    for rep in range(2):
+        r = run_pair(gpu_ctx, DESC, S.uniforms(), mesh, w, h, color_init=rep, gmesh=gm)
+        assert_bit_exact(r, f"{kind}, frame {rep}")
+    assert r["frags"] > 10000
