@@ -1744,7 +1744,9 @@ static void launch_setup_t(const FrameParams &p, hipStream_t s, bool batched, ui
             // Small meshes: 64 triangles a workgroup, so that the chip is not left idle
             // and a workgroup's pairs fit a round or two. With 256 against 64, us per
             // pass: 16 draws of 3000 triangles 295 / 275, a shadowed frame of 6400 54.9
-            // / 45.3, one of 29,700 21.7 / 21.5; at 262,144 triangles 36.6 / 41.3.
+            // / 45.3; tori of 32,768 triangles at 640, 1280 and 1920 columns 22.5 / 23.3,
+            // 22.0 / 21.5 and 25.1 / 24.6, of 76,800 23.6 / 24.1, 25.7 / 26.4 and 27.7 /
+            // 27.7, of 262,144 27.9 / 33.3, 32.8 / 36.9 and 34.5 / 38.9.
             q.tri_block = p.v0.n_tris <= kSmallMesh ? 64u : 256u;
             q.tri_blocks = blocks_of(p.v0.n_tris, q.tri_block);
             q.setup_blocks = q.tri_blocks + (vd_count(SH) > 0 ? blocks_of(nv, 256) : 0u);
